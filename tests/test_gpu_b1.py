@@ -176,6 +176,65 @@ def test_b1_backward_t8_bitwise(hip, oracle, n, k0, t8):
     assert np.array_equal(bits(gx), bits(ox))
 
 
+# The counting sort's tile (1024 connections) and wave edges, skewed sources
+# (long lists, many equal ids in a wave), the three LDS tile widths of dx
+# (n <= 2560, 5120, 10240), the radix-sort index (n > 8192) and half a block
+# of tokens (t8 = 8, 24).
+@pytest.mark.parametrize("n,k0,t8,skew", [(1, 1, 8, 1), (64, 16, 8, 1), (205, 5, 24, 9),
+                                          (1024, 3, 72, 50), (2560, 2, 16, 1), (2561, 2, 24, 4),
+                                          (5121, 1, 16, 1), (8192, 2, 8, 3), (8193, 2, 8, 3),
+                                          (10241, 1, 8, 1)])
+def test_b1_backward_index_edges_bitwise(hip, oracle, n, k0, t8, skew):
+    from sparrow_amd import ops
+    rng = np.random.default_rng(n + t8)
+    w = rng.standard_normal((n, k0)).astype(np.float32)
+    src = (rng.integers(0, n, size=(n, k0)) // skew).astype(np.uint32)
+    xt = rng.standard_normal((n, t8)).astype(np.float32)
+    dyt = rng.standard_normal((n, t8)).astype(np.float32)
+    dxt0 = rng.standard_normal((n, t8)).astype(np.float32)
+    dw0 = rng.standard_normal((n, k0)).astype(np.float32)
+    gx, gw = ops.b1_backward_t8(w, src, xt, dyt, dxt0, dw0)
+    ox, ow = oracle.b1_backward_t8(w, src, xt, dyt, dxt0, dw0)
+    assert np.array_equal(bits(gw), bits(ow)) and np.array_equal(bits(gx), bits(ox))
+    x, dy = xt[:, 0].copy(), dyt[:, 0].copy()
+    fx, _ = ops.b1_backward_dx(w, src, dy, dxt0[:, 0].copy())
+    assert np.array_equal(bits(fx), bits(oracle.b1_backward_dx(w, src, dy, dxt0[:, 0].copy())))
+
+
+def test_b1_backward_t8_unaligned_rows(hip, oracle):
+    """Activations 4 bytes past a 16-byte boundary take the kernels of single
+    floats: the same bits; an id past n is skipped and raises the guard."""
+    from sparrow_amd.conn import DeviceBuffer
+    n, k0, t8 = 96, 5, 16
+    rng = np.random.default_rng(3)
+    w = rng.standard_normal((n, k0)).astype(np.float32)
+    src = rng.integers(0, n, size=(n, k0)).astype(np.uint32)
+    rows = [rng.standard_normal((n, t8)).astype(np.float32) for _ in range(3)]
+    dw0 = rng.standard_normal((n, k0)).astype(np.float32)
+    for bad in (False, True):
+        s = src.copy()
+        ref_w, ref_s = w, src
+        if bad:
+            s[7, 2] = n
+            ref_w = w.copy()
+            ref_w[7, 2] = 0.0  # the connection adds nothing to dx (+-0)
+        bufs = [DeviceBuffer.from_array(np.concatenate([[np.float32(0)], r.ravel()]))
+                for r in rows]
+        dev = [DeviceBuffer.from_array(t) for t in (w, s, dw0)]
+        rc = hip.vmlm_hip_b1_backward_t8(dev[0].ptr, dev[1].ptr, bufs[0].ptr + 4, bufs[1].ptr + 4,
+                                         t8, n, k0, bufs[2].ptr + 4, dev[2].ptr, None)
+        assert rc == 0
+        assert hip.vmlm_hip_check_guards() == (9 if bad else 0)
+        gx = bufs[2].to_array((1 + n * t8,), np.float32)[1:].reshape(n, t8)
+        gw = dev[2].to_array((n, k0), np.float32)
+        ox, ow = oracle.b1_backward_t8(ref_w, ref_s, rows[0], rows[1], rows[2], dw0)
+        if bad:
+            ow[7, 2] = dw0[7, 2]
+        assert np.array_equal(bits(gw), bits(ow)) and np.array_equal(gx, ox)
+        for b in bufs + dev:
+            b.free()
+
+
 def test_b1_backward_guards(hip):
     from sparrow_amd import VmlmError, ops
     w = np.ones((4, 2), np.float32)
