@@ -264,11 +264,40 @@ static int download(void *host, const void *dev, size_t bytes, hipStream_t st) {
 
 static inline size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; }
 
+// Whether the one-launch GEMM over the caller's own rows (launch_gemm_direct)
+// is the faster way, against the times of the other paths (us, measured):
+//  * unpadded bf16 at m <= 16: the per-tile GEMV holds up to five rows' (term,
+//    row) pairs in one fragment and reads large tables at HBM rate, so the
+//    direct kernel only takes its small grids (1 x 2304 x 2304: 7.3 -> 6.3,
+//    equal near 20 us); with more rows it reads the activation again for every
+//    16 columns (16 x 122753 x 2304: 294 -> 108, 16 x 2304 x 2304: 14.3 -> 6.9);
+//  * unpadded int8 at m > 16: int8 rows, the GEMM, the slice reduction and the
+//    non-finite rows are four launches, 9 + 0.2 per k-step and the products
+//    at 500 TFLOP/s (17 x 2304 x 2304: 17.0 -> 7.2; 64 x 5760 x 2304: 21.1 ->
+//    15.8; 100 x 2304 x 5760: 27.6 -> 20.5); up to 128 rows, above which the
+//    row blocks of the int8 GEMM are full (300 x 5760 x 2304: 39 against 44);
+//  * else the padded weight copy, the term planes and the bf16 GEMM: 10, the
+//    copy at 4 TB/s, and 1.2 per k-step of one tile or the products at 230
+//    TFLOP/s (77 x 1537 x 1001 int8: 30.1 -> 6.6; 1000 x 1500 x 1100: 33.5 ->
+//    22.9; 333 x 1537 x 1536 bf16: 27.5 -> 15.3; 60 x 40509 x 2304 bf16 stays,
+//    66 to 78).
+static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
+    if (k == 0 || m > 4096 || n > (size_t)1 << 24 || k > (size_t)1 << 24) return false;
+    const double us = gemm_direct_us((int)m, (int)n, (int)k, wi8);
+    const double nk = (double)((k + 63) / 64), flop = 2.0 * m * n * k;
+    if (!padded && wi8) return m > 16 && m <= 128 && us < 9.0 + 0.2 * nk + flop / 500e6;
+    if (!padded && m <= 16) return m > 5 || us < 20.0;
+    const double steps = 1.2 * nk, prod = flop / 230e6;
+    const double copy = padded ? 2.0 * n * k * (wi8 ? 1 : 2) / 4e6 : 0.0;
+    return us < 10.0 + copy + (steps > prod ? steps : prod);
+}
+
 // int8 / bf16 weight GEMM on device operands: C[m,n] = A[m,k] . W[n,k]^T (* scale).
-// Pads K to a multiple of 128 when needed, then: int8 weights and m <= 16,
-// the wide k-split GEMV; int8 weights, m > 16 and K unpadded, int8 rows and
-// the int8 MFMA GEMM; otherwise A split into 3 bf16 terms and the GEMV kernel
-// (m <= 16) or the tiled bf16 MFMA GEMM.
+// int8 weights and m <= 16: the full-K GEMV (m <= FX_ROWS) or the wide k-split
+// GEMV; where it is faster (q_direct), one launch over the rows as they are;
+// int8 weights, m > 16 and K a multiple of 128, int8 rows and the int8 MFMA
+// GEMM; otherwise A split into 3 bf16 terms, K padded to a multiple of 128,
+// and a GEMV kernel (m <= 16) or the tiled bf16 MFMA GEMM.
 // Temporaries come from `stg`: the stream's arena (Stage) or the fixed
 // scratch array of the allocation-free entry point (ScratchBump). Wsw, when
 // given, is a swizzled copy of int8 W (launch_swizzle_w) that the caller
@@ -280,15 +309,48 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
     if (m == 0 || n == 0) return VMLM_OK;
     const size_t esz = wi8 ? 1 : 2;
     const size_t Kp = round_up(k == 0 ? 1 : k, 128);  // one 128-byte GEMV chunk covers 128 k
+    const bool padded = Kp != k || ((uintptr_t)W & 15);
     const void *Wd = W;
-    if (Kp != k || ((uintptr_t)W & 15)) {
+    if (padded) {
         // the padded weight copy is a device copy: refused up front while the
-        // stream is being captured, so a capture never records it
+        // stream is being captured, so a capture never records it (whether or
+        // not this shape takes it)
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         VMLM_HIP_CHECK(hipStreamIsCapturing(st, &cs));
         if (cs != hipStreamCaptureStatusNone)
             return fail(VMLM_ERR_UNIMPL, "q8/bf16 GEMM with K %% 128 != 0 or unaligned weights "
                                          "stages a padded weight copy and cannot be captured");
+    }
+    const bool few = wi8 && m <= 16 && !padded && ((uintptr_t)a & 15) == 0;
+    if (!few && q_direct(wi8, padded, m, n, k)) {
+        // the fixed scratch keeps its limit of shapes, whichever path they take
+        if constexpr (!std::is_same<WS, Stage>::value) {
+            if (padded) stg.template alloc<uint8_t>(n * Kp * esz);
+            if (!padded && wi8 && m > 16 && k <= 8192) {
+                stg.template alloc<int8_t>(q8_rows_bytes(m, k));
+                stg.template alloc<float>(m);
+                const size_t gw = gemm_i8_work_floats((int)m, (int)n, (int)k);
+                if (gw) stg.template alloc<float>(gw);
+            } else {
+                stg.template alloc<uint16_t>(3 * m * Kp);
+            }
+            STAGE_OK(stg);
+        }
+        GemmDirectArgs d;
+        d.A = a;
+        d.lda = k;
+        d.W = W;
+        d.w_int8 = wi8;
+        d.ldw = k;
+        d.scale = scale;
+        d.C = c;
+        d.ldc = n;
+        d.M = (int)m;
+        d.N = (int)n;
+        d.K = (int)k;
+        return launch_gemm_direct(d, st);
+    }
+    if (padded) {
         uint8_t *wp = stg.template alloc<uint8_t>(n * Kp * esz);
         STAGE_OK(stg);
         int rc0 = launch_fill_zero(wp, n * Kp * esz, st);

@@ -223,6 +223,23 @@ int q8_gemm_vm(const float *a, const int8_t *q, const int8_t *wsw, const float *
 // int8 [N][K] row-major -> [N/16][K/64][64 lanes][16 B] MFMA-operand order.
 int launch_swizzle_w(const int8_t *src, int8_t *dst, int N, int K, hipStream_t st);
 
+// C[M,N] = A[M,K] . W[N,K]^T (* scale[n]) straight from the caller's f32 rows
+// and weight rows, any K and alignment, in one launch (k_direct.hip).
+// gemm_direct_us: about how long it takes.
+struct GemmDirectArgs {
+    const float *A = nullptr;
+    size_t lda = 0;
+    const void *W = nullptr;  // int8 or bf16 bits [N][ldw]
+    bool w_int8 = true;
+    size_t ldw = 0;
+    const float *scale = nullptr;
+    float *C = nullptr;
+    size_t ldc = 0;
+    int M = 0, N = 0, K = 0;
+};
+double gemm_direct_us(int M, int N, int K, bool w_int8);
+int launch_gemm_direct(const GemmDirectArgs &a, hipStream_t st);
+
 // Tiled MFMA GEMM for M > 16: C[M,N] = A[M,K] . W[N,K]^T (* scale[n]).
 struct GemmArgs {
     const void *W = nullptr;

@@ -184,3 +184,64 @@ def test_gemm_int8_many_tiles_exact(dev, m, n):
     ref = a[:m - 1].astype(np.float64) @ q.astype(np.float64).T
     np.testing.assert_array_equal(got[:m - 1].astype(np.float64), ref)
     assert np.isnan(got[m - 1]).all()
+
+
+def direct_case(rng, m, n, k, int8):
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    if int8:
+        w = rng.integers(-127, 128, size=(n, k), dtype=np.int8)
+        return a, w, w.astype(np.float64), rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+    u = rng.standard_normal((n, k), dtype=np.float32).view(np.uint32) & np.uint32(0xffff0000)
+    return a, (u >> np.uint32(16)).astype(np.uint16), u.view(np.float32).astype(np.float64), None
+
+
+# One launch over the rows as they are: K below, at and past the 64-wide blocks
+# and the eight runs, rows and columns at the edges of each tile (16 x 16, 16 x
+# 32, 16 x 64, 32 x 32, 32 x 64) and operands at any byte or float alignment.
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (2, 17, 63), (16, 33, 65), (17, 40, 577),
+                                   (33, 2050, 513), (77, 1537, 1001), (100, 2304, 5760),
+                                   (300, 1000, 1000), (1000, 1500, 100), (12, 9000, 1536)])
+def test_gemm_direct_edges(dev, m, n, k, int8):
+    """Against float64. A result is at most ceil(K / 64 / 4) blocks of two
+    MFMAs and three terms in one chain, each MFMA adding 32 products in f32,
+    then at most eight waves: the error is within (32 * 6 * ceil(K / 256) + 10)
+    roundings of 2^-24 of sum |a w|."""
+    rng = np.random.default_rng(m + n + k)
+    a, w, w64, s = direct_case(rng, m, n, k, int8)
+    ref = a.astype(np.float64) @ w64.T
+    bound = (192 * -(-k // 256) + 10) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(w64).T)
+    if int8:
+        ref, bound = ref * s, bound * s
+    c = dev.empty(m * n * 4)
+    for skew in (0, 1):  # rows as allocated, then off by one element (f32 4 bytes, weights 1 or 2)
+        off = skew * w.itemsize
+        da = dev.up(np.concatenate([np.zeros(4 * skew, np.uint8), a.view(np.uint8).ravel()]))
+        dw = dev.up(np.concatenate([np.zeros(off, np.uint8), w.view(np.uint8).ravel()]))
+        pa, pw = C.c_void_p(da.value + 4 * skew), C.c_void_p(dw.value + off)
+        if int8:
+            dev.check(dev.lib.vmlm_hip_gemm_nt_int8(pa, pw, dev.up(s), c, m, n, k, None))
+        else:
+            dev.check(dev.lib.vmlm_hip_gemm_nt_bf16(pa, pw, c, m, n, k, None))
+        got = dev.down(c, (m, n), np.float32).astype(np.float64)
+        assert (np.abs(got - ref) <= bound).all()
+
+
+def test_gemm_direct_infinite_and_nan_rows(dev):
+    """A row with an infinity or a NaN takes the split that keeps them in the
+    first term: +-inf by the weight's sign, NaN at a zero weight or a NaN."""
+    rng = np.random.default_rng(2)
+    m, n, k = 20, 70, 130
+    a, w, w64, s = direct_case(rng, m, n, k, True)
+    a[3, 129] = np.inf
+    a[4, 5] = np.nan
+    a[19, 0] = -np.inf
+    with np.errstate(invalid="ignore"):
+        ref = (a.astype(np.float64) @ w64.T) * s
+    c = dev.empty(m * n * 4)
+    dev.check(dev.lib.vmlm_hip_gemm_nt_int8(dev.up(a), dev.up(w), dev.up(s), c, m, n, k, None))
+    got = dev.down(c, (m, n), np.float32)
+    for f in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(f(got), f(ref))
+    ok = np.isfinite(ref)
+    assert np.abs(got[ok] - ref[ok]).max() <= 1e-5 * np.sqrt(np.mean(ref[ok] ** 2))
