@@ -301,13 +301,22 @@ __device__ __forceinline__ float act_scalar(float x, int kind) {
 
 // core/src/interp.rs:1183-1221: the rotation of RoPE component i at position
 // `pos` (a function of (pos, i) only, so rows at one position share it) ...
-__device__ __forceinline__ void rope_angle(float pos, int i, float step, float *si, float *co) {
+// (rope_freq: what depends on the component alone)
+__device__ __forceinline__ void rope_freq(int i, float step, float *inv, float *period) {
     const float TWO_PI = 6.2831855f;
-    float inv = exp_f((float)i * step);
-    float period = TWO_PI / inv;
+    *inv = exp_f((float)i * step);
+    *period = TWO_PI / *inv;
+}
+__device__ __forceinline__ void rope_angle_at(float pos, float inv, float period, float *si,
+                                              float *co) {
     float pr = period >= 1.0e6f ? pos : pos - period * floor_f(pos / period);
     float ang = pr * inv;
     sincos_f(ang, si, co);
+}
+__device__ __forceinline__ void rope_angle(float pos, int i, float step, float *si, float *co) {
+    float inv, period;
+    rope_freq(i, step, &inv, &period);
+    rope_angle_at(pos, inv, period, si, co);
 }
 // ... and one rotated pair
 __device__ __forceinline__ void rope_pair(float x1, float x2, float pos, int i, float step,
@@ -368,6 +377,41 @@ __device__ __forceinline__ float wave_sum_dpp(float v) {
     const float r2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
     const float r3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 48));
     return (r0 + r1) + (r2 + r3);
+}
+
+// ------------------------------------------------------------------ LDS copies
+// s_waitcnt immediate (gfx9 encoding) that waits for the vector-memory
+// counter to drop to n and leaves the other counters unconstrained.
+constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
+
+// One 16-byte-per-lane copy from global memory into LDS: lane i's 16 bytes
+// at gptr land at LDS byte address lds_base + 16 * i (lds_base wave-uniform).
+// Issued as inline assembly so that the compiler does not order every later
+// LDS read behind it; the callers wait for the copies with explicit vmcnt
+// waits and publish them with barriers. m0 is not used by anything else in
+// the kernels that use these.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved; nothing else here uses it
+__device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+                 :
+                 : "v"(gptr), "s"(lds_base)
+                 : "memory", "m0");
+}
+
+// The same copy with a wave-uniform base held in SGPRs (sbase) and a 32-bit
+// per-lane byte offset: one VGPR per distinct offset instead of a 64-bit
+// address per copy.
+__device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff), "s"(sbase), "s"(lds_base)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+__device__ __forceinline__ uint32_t lds_addr(const void *p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)p;
 }
 
 inline unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }

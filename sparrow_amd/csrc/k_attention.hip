@@ -181,20 +181,27 @@ int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n
 // each exact, accumulated in f32 by v_mfma_f32_16x16x32_bf16: relative error
 // ~2^-16, well inside the 1e-4 * RMS contract of the attention composition,
 // and a one-key softmax row returns its V row exactly. A workgroup owns 64
-// queries of one head (wave w: queries 16w..16w+15) and walks the key blocks
-// of 64 up to the diagonal: K is staged as [key][dim] terms, V transposed as
-// [dim][key] terms.
+// or 128 queries of one head (16 or 32 a wave) and walks the key blocks of 64 up
+// to the diagonal: K is staged as [key][dim] terms, V transposed as [dim][key]
+// terms.
 //
 // Both products are computed transposed, S^T = K Q^T and O^T += V^T P^T, so
 // that the accumulator layout (lane (g, r): rows 4g..4g+3 of column r) puts
 // one query (column r) in each lane: its scores for keys 16j + 4g + i are
 // exactly the B-operand fragment of the next product once the key slots of a
-// 32-key step are taken in the order (32m + 4g + i, 32m + 16 + 4g + i), and V
-// is read in the same order. The probabilities never leave registers; the
+// 32-key step are taken in the order (32m + 4g + i, 32m + 16 + 4g + i), and V^T
+// is laid out in that order. The probabilities never leave registers; the
 // running max / sum of a query live in its lane (the four lanes g of a query
 // exchange partial max / sum with permlane swaps).
 constexpr int AT_B = 64;   // query / key block
-constexpr int AT_LD = 72;  // bf16 elements per LDS row (64 + 8)
+// The terms of one key block are a tile of 5 x 64 rows of 64 bf16 (40 KiB): two
+// term planes of K [key][dim], three of V^T [dim][key]. A row's 16-byte piece c
+// sits in slot c ^ (row / 2 % 8) (fragment reads of 16 rows spread over the
+// banks), and the keys of a V^T row are in the order that the probabilities'
+// fragments have them: piece 4 st + g holds keys 32 st + 4g .. + 3 and
+// 32 st + 16 + 4g .. + 3, so a fragment is one 16-byte read.
+constexpr int AT_TILE = 5 * AT_B * AT_B;  // bf16 elements
+__device__ __forceinline__ int at_piece(int row, int c) { return 8 * (c ^ ((row >> 1) & 7)); }
 
 // DPP lane moves inside a row of 16 lanes (row_mirror: lane i <- 15 - i;
 // row_half_mirror: i <- 7 - i within each 8; quad_perm [3,2,1,0] and
@@ -273,23 +280,26 @@ __device__ __forceinline__ void split8x3(const float (&x)[8], u32x4 &t0, u32x4 &
 // One workgroup per (query block, head, sequence); sequences at strides
 // sin / sout (elements) along grid z. The longest causal rows go first.
 struct PrefillParams {
-    const uint16_t *Qt, *Kt, *Vt;  // bf16 term planes written by attn_qkv_prep_kernel
+    const uint16_t *Qt, *KV;  // written by attn_qkv_prep_kernel
     float *O;
     size_t sout;
     int S, Sp, ldo, causal, nqb, H;
-    int o_vec;  // O rows 16-byte aligned: float4 stores
-    float scale;
+    int nseq;
+    int o_vec;     // O rows 16-byte aligned: float4 stores
+    float scale2;  // score scale times log2(e)
 };
 
 // Q, K and V of every (sequence, head) as bf16 term planes, rows padded to Sp
 // (a multiple of 64) with zeros:
-//   Qt[z][t][h][row][64], Kt[z][t][h][row][64]  (t < 2; rotated here when
-//                                               rope is set)
-//   Vt[z][t][h][dim][Sp]                        (t < 3; V transposed)
-// so that the attention kernel loads its Q fragments and stages each key
-// block with 16-byte copies. One workgroup per (64-row block, head,
-// sequence); thread (row, c) rotates RoPE pairs 2c and 2c + 1 of its Q and K
-// rows with one angle evaluation per pair (Q and K share the position).
+//   Qt[z][t][h][row][64]          (t < 2; rotated here when rope is set)
+//   KV[z][h][key block][AT_TILE]  (the block's K and V^T tile)
+// so that the attention kernel loads its Q fragments, and copies a key block
+// into LDS as it is. One workgroup per (64-row block, head, sequence); thread
+// (row, c) rotates RoPE pairs 2c and 2c + 1 of its Q and K rows with one angle
+// evaluation per pair (Q and K share the position; the pairs' frequencies are
+// evaluated once a workgroup). Several heads a workgroup, one angle for all of
+// them, was slower (13.2 -> 14.7 us at 36 heads, 1000 rows: twice the registers,
+// half the waves).
 // With kc / vc the rotated K rows and the raw V rows also go to a KV cache
 // [sequence][head][hs][64] f32 at positions 0 .. S-1 (the decoder's prefill).
 // With pks > 0, Q, K and V point into slice 0 of pks k-slices pst floats
@@ -297,7 +307,7 @@ struct PrefillParams {
 // (sq, sk, sv), as the slice reduction would have written it.
 struct QKVPrepParams {
     const float *Q, *K, *V;
-    uint16_t *Qt, *Kt, *Vt;
+    uint16_t *Qt, *KV;
     float *kc, *vc;
     size_t sin;
     int S, Sp, ld, H, rope, hs;
@@ -307,12 +317,35 @@ struct QKVPrepParams {
     const float *sq, *sk, *sv;
 };
 __global__ __launch_bounds__(1024) void attn_qkv_prep_kernel(QKVPrepParams p) {
+    __shared__ float vs[AT_B][AT_B + 1];
+    __shared__ float2 freq[32];  // rope_freq of each pair
     const int h = blockIdx.y, z = blockIdx.z, tid = threadIdx.x;
     const int k0 = blockIdx.x * AT_B;
     const size_t plane = (size_t)p.H * p.Sp * 64;
+    uint16_t *tile = p.KV + (((size_t)z * p.H + h) * (p.Sp / AT_B) + blockIdx.x) * AT_TILE;
+    if (p.rope && tid < 32) rope_freq(tid, p.rope_step, &freq[tid].x, &freq[tid].y);
+    const int lr = tid >> 4, c = tid & 15, row = k0 + lr, rr = min(row, p.S - 1);
+    const size_t src = z * p.sin + (size_t)rr * p.ld + h * 64 + 2 * c;
     {
-        const int row = k0 + (tid >> 4), c = tid & 15, rr = min(row, p.S - 1);
-        const size_t src = z * p.sin + (size_t)rr * p.ld + h * 64 + 2 * c;
+        // V rows into LDS as float4: dims 4c .. 4c + 3
+        const size_t vsrc = src + 2 * c;
+        float4 x = *(const float4 *)(p.V + vsrc);
+        if (p.pks) {
+            for (int s = 1; s < p.pks; ++s) {
+                const float4 t = *(const float4 *)(p.V + (size_t)s * p.pst + vsrc);
+                x = make_float4(x.x + t.x, x.y + t.y, x.z + t.z, x.w + t.w);
+            }
+            const float4 sc = *(const float4 *)(p.sv + h * 64 + 4 * c);
+            x = make_float4(x.x * sc.x, x.y * sc.y, x.z * sc.z, x.w * sc.w);
+        }
+        const bool ok = row < p.S;
+        if (ok && p.vc) *(float4 *)(p.vc + (((size_t)z * p.H + h) * p.hs + row) * 64 + 4 * c) = x;
+        vs[lr][4 * c] = ok ? x.x : 0.0f;
+        vs[lr][4 * c + 1] = ok ? x.y : 0.0f;
+        vs[lr][4 * c + 2] = ok ? x.z : 0.0f;
+        vs[lr][4 * c + 3] = ok ? x.w : 0.0f;
+    }
+    {
         auto ld2 = [&](const float *b, const float *sc, int off) {
             float2 v = *(const float2 *)(b + src + off);
             if (p.pks) {
@@ -328,13 +361,14 @@ __global__ __launch_bounds__(1024) void attn_qkv_prep_kernel(QKVPrepParams p) {
         };
         float2 q1 = ld2(p.Q, p.sq, 0), q2 = ld2(p.Q, p.sq, 32);
         float2 k1 = ld2(p.K, p.sk, 0), k2 = ld2(p.K, p.sk, 32);
+        __syncthreads();  // freq and the V rows are in LDS
         if (p.rope) {
             const float fpos = p.pos0 + (float)rr;
             float si, co, a, b;
-            rope_angle(fpos, 2 * c, p.rope_step, &si, &co);
+            rope_angle_at(fpos, freq[2 * c].x, freq[2 * c].y, &si, &co);
             a = q1.x * co - q2.x * si, b = q1.x * si + q2.x * co, q1.x = a, q2.x = b;
             a = k1.x * co - k2.x * si, b = k1.x * si + k2.x * co, k1.x = a, k2.x = b;
-            rope_angle(fpos, 2 * c + 1, p.rope_step, &si, &co);
+            rope_angle_at(fpos, freq[2 * c + 1].x, freq[2 * c + 1].y, &si, &co);
             a = q1.y * co - q2.y * si, b = q1.y * si + q2.y * co, q1.y = a, q2.y = b;
             a = k1.y * co - k2.y * si, b = k1.y * si + k2.y * co, k1.y = a, k2.y = b;
         }
@@ -344,165 +378,158 @@ __global__ __launch_bounds__(1024) void attn_qkv_prep_kernel(QKVPrepParams p) {
             *(float2 *)kr = k1;
             *(float2 *)(kr + 32) = k2;
         }
-        const size_t dst = ((size_t)z * 2 * p.H + h) * p.Sp * 64 + (size_t)row * 64 + 2 * c;
-        auto put = [&](uint16_t *base, float2 lo, float2 hi) {
+        // dims 2c, 2c + 1 (lo) and 32 + 2c, 33 + 2c (hi), the two terms a plane apart
+        auto put = [&](uint16_t *l, uint16_t *u, size_t pl, float2 lo, float2 hi) {
             const uint32_t l0 = bf16x2_rne_bits(lo.x, lo.y), h0 = bf16x2_rne_bits(hi.x, hi.y);
-            *(uint32_t *)(base + dst) = l0;
-            *(uint32_t *)(base + dst + 32) = h0;
-            *(uint32_t *)(base + dst + plane) =
-                bf16x2_rne_bits(lo.x - bf16_lo_f32(l0), lo.y - bf16_hi_f32(l0));
-            *(uint32_t *)(base + dst + plane + 32) =
-                bf16x2_rne_bits(hi.x - bf16_lo_f32(h0), hi.y - bf16_hi_f32(h0));
+            *(uint32_t *)l = l0;
+            *(uint32_t *)u = h0;
+            *(uint32_t *)(l + pl) = bf16x2_rne_bits(lo.x - bf16_lo_f32(l0), lo.y - bf16_hi_f32(l0));
+            *(uint32_t *)(u + pl) = bf16x2_rne_bits(hi.x - bf16_lo_f32(h0), hi.y - bf16_hi_f32(h0));
         };
-        put(p.Qt, q1, q2);
-        put(p.Kt, k1, k2);
+        uint16_t *qd = p.Qt + ((size_t)z * 2 * p.H + h) * p.Sp * 64 + (size_t)row * 64 + 2 * c;
+        put(qd, qd + 32, plane, q1, q2);
+        uint16_t *kd = tile + lr * AT_B + 2 * (c & 3);
+        put(kd + at_piece(lr, c >> 2), kd + at_piece(lr, 4 + (c >> 2)), AT_B * AT_B, k1, k2);
     }
-    {
-        // V transposed through LDS: rows read as float4 (thread: row tid / 16,
-        // dims 4 (tid % 16) ..), then thread (dim, key octet) of the first 512
-        // splits 8 consecutive keys and writes each term as one 16-byte piece
-        __shared__ float vs[AT_B][AT_B + 1];
-        {
-            const int row = k0 + (tid >> 4), d0 = 4 * (tid & 15);
-            const size_t vsrc = z * p.sin + (size_t)min(row, p.S - 1) * p.ld + h * 64 + d0;
-            float4 x = *(const float4 *)(p.V + vsrc);
-            if (p.pks) {
-                for (int s = 1; s < p.pks; ++s) {
-                    const float4 t = *(const float4 *)(p.V + (size_t)s * p.pst + vsrc);
-                    x = make_float4(x.x + t.x, x.y + t.y, x.z + t.z, x.w + t.w);
-                }
-                const float4 sc = *(const float4 *)(p.sv + h * 64 + d0);
-                x = make_float4(x.x * sc.x, x.y * sc.y, x.z * sc.z, x.w * sc.w);
-            }
-            const bool ok = row < p.S;
-            if (ok && p.vc) *(float4 *)(p.vc + (((size_t)z * p.H + h) * p.hs + row) * 64 + d0) = x;
-            vs[tid >> 4][d0] = ok ? x.x : 0.0f;
-            vs[tid >> 4][d0 + 1] = ok ? x.y : 0.0f;
-            vs[tid >> 4][d0 + 2] = ok ? x.z : 0.0f;
-            vs[tid >> 4][d0 + 3] = ok ? x.w : 0.0f;
-        }
-        __syncthreads();
-        if (tid < 512) {
-            const int dim = tid >> 3, kg = tid & 7;
-            float x[8];
+    // V transposed: thread (dim, piece) of the first 512 splits the piece's 8
+    // keys and writes each term as one 16-byte piece
+    if (tid < 512) {
+        const int dim = tid >> 3, kg = tid & 7, key = 32 * (kg >> 2) + 4 * (kg & 3);
+        float x[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] = vs[8 * kg + i][dim];
-            u32x4 t0, t1, t2;
-            split8x3(x, t0, t1, t2);
-            uint16_t *vt =
-                p.Vt + ((size_t)z * 3 * p.H + h) * 64 * p.Sp + (size_t)dim * p.Sp + k0 + 8 * kg;
-            *(u32x4 *)vt = t0;
-            *(u32x4 *)(vt + plane) = t1;
-            *(u32x4 *)(vt + 2 * plane) = t2;
-        }
+        for (int i = 0; i < 8; ++i) x[i] = vs[key + 12 * (i >> 2) + i][dim];
+        u32x4 t0, t1, t2;
+        split8x3(x, t0, t1, t2);
+        uint16_t *vt = tile + 2 * AT_B * AT_B + dim * AT_B + at_piece(dim, kg);
+        *(u32x4 *)vt = t0;
+        *(u32x4 *)(vt + AT_B * AT_B) = t1;
+        *(u32x4 *)(vt + 2 * AT_B * AT_B) = t2;
     }
 }
 
-// One key block of the prefill attention for the wave's 16 queries: S^T =
+// One key block of the prefill attention for the wave's NQ x 16 queries: S^T =
 // K Q^T over the block's 64 keys (two bf16 terms of K and of Q), the online
 // softmax update of (m, l, o), then O^T += V^T P^T (three terms of V, two of
-// P). Ks / Vt hold the block's terms in LDS; lane (g, r) owns query qa.
-__device__ __forceinline__ void prefill_block(const uint16_t (*Ks)[AT_B][AT_LD],
-                                              const uint16_t (*Vt)[64][AT_LD],
-                                              const u32x4 (&aq)[2][2], int k0, int qa, int S,
-                                              int causal, float scale, float &m, float &l,
-                                              f32x4 (&o)[4]) {
+// P). T: the block's tile in LDS; lane (g, r) owns queries qa + 16 n. scale2 is
+// the score scale times log2(e): the maximum m and the exponents are in base
+// 2. Only a block that crosses the diagonal or the last key masks.
+template <int NQ>
+__device__ __forceinline__ void prefill_block(const uint16_t (*T)[AT_B][AT_B],
+                                              const u32x4 (&aq)[NQ][2][2], int k0, int qa, int S,
+                                              int causal, float scale2, float (&m)[NQ],
+                                              float (&l)[NQ], f32x4 (&o)[NQ][4]) {
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
     // S^T: block j = keys 16j..16j+15; lane (g, r): keys 16j + 4g + i of
     // query q0 + r. The four blocks' MFMA chains are interleaved.
-    f32x4 sc[4];
+    f32x4 sc[NQ][4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < NQ; ++n)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sc[n][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
         u32x4 b0[4], b1[4];
+        const int at = at_piece(r, 4 * sl + g);  // rows 16 j + r swizzle alike
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            b0[j] = *(const u32x4 *)&Ks[0][16 * j + r][sl * 32 + g * 8];
-            b1[j] = *(const u32x4 *)&Ks[1][16 * j + r][sl * 32 + g * 8];
+            b0[j] = *(const u32x4 *)&T[0][16 * j + r][at];
+            b1[j] = *(const u32x4 *)&T[1][16 * j + r][at];
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc[j] = mfma_b(b0[j], aq[sl][0], sc[j]);
+        for (int t = 0; t < 2; ++t) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc[j] = mfma_b(b1[j], aq[sl][0], sc[j]);
+            for (int n = 0; n < NQ; ++n)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc[j] = mfma_b(b0[j], aq[sl][1], sc[j]);
+                for (int j = 0; j < 4; ++j) sc[n][j] = mfma_b(b0[j], aq[n][sl][t], sc[n][j]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) sc[j] = mfma_b(b1[j], aq[sl][1], sc[j]);
+            for (int n = 0; n < NQ; ++n)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) sc[n][j] = mfma_b(b1[j], aq[n][sl][t], sc[n][j]);
+        }
     }
-    float mx = -INFINITY;
+    const int q0 = __builtin_amdgcn_readfirstlane(qa);  // lane 0: r = 0, the wave's first query
+    const bool mask = k0 + AT_B > S || (causal && k0 + AT_B - 1 > q0);
+    u32x4 pb[NQ][2][2];  // P^T fragments of the two 32-key steps, two terms
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int n = 0; n < NQ; ++n) {
+        if (mask) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int ka = k0 + 16 * j + 4 * g + i;
-            const bool valid = ka < S && (!causal || ka <= qa);
-            sc[j][i] = valid ? sc[j][i] * scale : -INFINITY;
-            mx = fmaxf(mx, sc[j][i]);
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int ka = k0 + 16 * j + 4 * g + i;
+                    const bool valid = ka < S && (!causal || ka <= qa + 16 * n);
+                    sc[n][j][i] = valid ? sc[n][j][i] * scale2 : -INFINITY;
+                }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sc[n][j][i] = sc[n][j][i] * scale2;
         }
-    mx = fmaxf(mx, lane_xor16(mx));
-    mx = fmaxf(mx, lane_xor32(mx));
-    const float mn = fmaxf(m, mx);
-    const float alpha = m == -INFINITY ? 0.0f : __expf(m - mn);
-    float pv[4][4], rs = 0.0f;
+        float mx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            pv[j][i] = sc[j][i] == -INFINITY ? 0.0f : __expf(sc[j][i] - mn);
-            rs += pv[j][i];
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[n][j][i]);
+        mx = fmaxf(mx, lane_xor16(mx));
+        mx = fmaxf(mx, lane_xor32(mx));
+        const float mn = fmaxf(m[n], mx);
+        // no finite score yet: exponents of -inf - 0 are 0 (not -inf - -inf = NaN)
+        const float mref = mn == -INFINITY ? 0.0f : mn;
+        const float alpha = __builtin_amdgcn_exp2f(m[n] - mref);
+        float rs = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sc[n][j][i] = __builtin_amdgcn_exp2f(sc[n][j][i] - mref);
+                rs += sc[n][j][i];
+            }
+        rs += lane_xor16(rs);
+        rs += lane_xor32(rs);
+        l[n] = l[n] * alpha + rs;
+        m[n] = mn;
+#pragma unroll
+        for (int jd = 0; jd < 4; ++jd)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[n][jd][i] *= alpha;
+        // slots 8g..8g+7 hold keys 32 st + 4g + i and 32 st + 16 + 4g + i
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            const f32x4 a = sc[n][2 * st], b = sc[n][2 * st + 1];
+            const float x[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+            split8(x, pb[n][st][0], pb[n][st][1]);
         }
-    rs += lane_xor16(rs);
-    rs += lane_xor32(rs);
-    l = l * alpha + rs;
-    m = mn;
-#pragma unroll
-    for (int jd = 0; jd < 4; ++jd)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o[jd][i] *= alpha;
-    // P^T fragments of the two 32-key steps: slots 8g..8g+7 hold keys
-    // 32 st + 4g + i and 32 st + 16 + 4g + i
-    u32x4 pb[2][2];
-#pragma unroll
-    for (int st = 0; st < 2; ++st) {
-        const float x[8] = {pv[2 * st][0],     pv[2 * st][1],     pv[2 * st][2],
-                            pv[2 * st][3],     pv[2 * st + 1][0], pv[2 * st + 1][1],
-                            pv[2 * st + 1][2], pv[2 * st + 1][3]};
-        split8(x, pb[st][0], pb[st][1]);
     }
     // O^T[d][q] += V^T[d][key] P^T[key][q]: A = V^T rows (dim 16 jd + r)
     // at the same key slots; the four dim blocks' chains interleaved
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
         u32x4 va[3][4];
+        const int at = at_piece(r, 4 * st + g);
 #pragma unroll
         for (int t = 0; t < 3; ++t)
 #pragma unroll
-            for (int jd = 0; jd < 4; ++jd) {
-                const uint16_t *row = &Vt[t][16 * jd + r][32 * st + 4 * g];
-                const uint2 lo = *(const uint2 *)row, hi = *(const uint2 *)(row + 16);
-                va[t][jd] = u32x4{lo.x, lo.y, hi.x, hi.y};
-            }
+            for (int jd = 0; jd < 4; ++jd) va[t][jd] = *(const u32x4 *)&T[2 + t][16 * jd + r][at];
 #pragma unroll
-        for (int jd = 0; jd < 4; ++jd) o[jd] = mfma_b(va[0][jd], pb[st][0], o[jd]);
+        for (int e = 0; e < 5; ++e)  // v0 p0, v1 p0, v2 p0, v0 p1, v1 p1
 #pragma unroll
-        for (int jd = 0; jd < 4; ++jd) o[jd] = mfma_b(va[1][jd], pb[st][0], o[jd]);
+            for (int n = 0; n < NQ; ++n)
 #pragma unroll
-        for (int jd = 0; jd < 4; ++jd) o[jd] = mfma_b(va[2][jd], pb[st][0], o[jd]);
-#pragma unroll
-        for (int jd = 0; jd < 4; ++jd) o[jd] = mfma_b(va[0][jd], pb[st][1], o[jd]);
-#pragma unroll
-        for (int jd = 0; jd < 4; ++jd) o[jd] = mfma_b(va[1][jd], pb[st][1], o[jd]);
+                for (int jd = 0; jd < 4; ++jd)
+                    o[n][jd] = mfma_b(va[e % 3][jd], pb[n][st][e / 3], o[n][jd]);
     }
 }
 
 // lane (g, r): query qa, dims 16 jd + 4g .. +3
 __device__ __forceinline__ void prefill_store(const f32x4 (&o)[4], float l, int qa, int S,
-                                              float *O, size_t sout, int ldo, int o_vec, int h) {
+                                              float *O, size_t sout, int ldo, int o_vec, int h,
+                                              int z) {
     const int g = (threadIdx.x & 63) >> 4;
     if (qa >= S) return;
     const float inv = 1.0f / l;
-    float *orow = O + blockIdx.z * sout + (size_t)qa * ldo + h * 64 + 4 * g;
+    float *orow = O + z * sout + (size_t)qa * ldo + h * 64 + 4 * g;
 #pragma unroll
     for (int jd = 0; jd < 4; ++jd) {
         const float4 v = make_float4(o[jd][0] * inv, o[jd][1] * inv, o[jd][2] * inv, o[jd][3] * inv);
@@ -517,73 +544,140 @@ __device__ __forceinline__ void prefill_store(const f32x4 (&o)[4], float l, int 
     }
 }
 
-__global__ __launch_bounds__(256, 2) void attn_prefill_kernel(PrefillParams P) {
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[2][AT_B][AT_LD];   // [term][key][dim]
-    __shared__ __attribute__((aligned(16))) uint16_t Vt[3][64][AT_LD];     // [term][dim][key]
+// The (query block, head, sequence) of a workgroup, from a one-dimensional
+// grid of prefill_grid() workgroups. Workgroup i runs on XCD i % 8. Causal
+// query blocks take 1 to nqb key blocks, so the heaviest come first, and with
+// neighbouring workgroups on neighbouring query blocks (grid x = query block)
+// XCD 0 would get the heaviest of every head: 1.4 times the mean at 16 query
+// blocks. Here the U = H * nseq (head, sequence) pairs are dealt to the XCDs
+// where that is even (a multiple of 8, or many), so that a pair's K and V stay
+// in one XCD's L2; else consecutive workgroups take consecutive pairs of one
+// query block. False: past the end (the deal's remainder).
+__host__ __device__ inline bool prefill_dealt(int U) { return U % 8 == 0 || U >= 32; }
+__host__ __device__ inline long long prefill_grid(int nqb, int U) {
+    return (long long)nqb * (prefill_dealt(U) ? (U + 7) / 8 * 8 : U);
+}
+__device__ __forceinline__ bool prefill_unit(int nqb, int H, int nseq, int causal, int &qb, int &h,
+                                             int &z) {
+    const int U = H * nseq, id = (int)blockIdx.x;
+    int qi, u;
+    if (prefill_dealt(U)) {
+        const int xcd = id & 7, j = id >> 3, per = (U + 7 - xcd) / 8;
+        qi = j / per;
+        u = xcd + 8 * (j - qi * per);
+        if (qi >= nqb) return false;
+    } else {
+        qi = id / U;
+        u = id - qi * U;
+    }
+    qb = causal ? nqb - 1 - qi : qi;
+    z = u / H;
+    h = u - z * H;
+    return true;
+}
+
+// A workgroup owns 64 NQ queries, 16 NQ a wave: a fragment read from LDS, whose
+// reads bound the kernel (54 % of its cycles at 16 queries a wave), serves NQ
+// tiles. Two groups of four waves take alternate key blocks and merge their
+// (max, sum, O) at the end: the last rows' query blocks are otherwise one serial
+// chain of all key blocks, which bounds the launch. Up to four key blocks stay
+// with the first group (the one-launch kernel's sum, the same bits). Each group
+// copies its tiles straight into its two LDS stages, the next one while the
+// current one is consumed. 36 heads, 1000 causal rows, with the
+// prep launch: 83.6 -> 46 us (2048 rows 244 -> 125).
+constexpr int AT_SPLIT = 4;
+template <int NQ, int NG>
+__global__ __launch_bounds__(256 * NG, 2) void attn_prefill_kernel(PrefillParams P) {
+    __shared__ __attribute__((aligned(1024))) uint16_t tiles[NG][2][5][AT_B][AT_B];  // [group][stage]
     const int S = P.S, causal = P.causal;
-    const int h = blockIdx.y, z = blockIdx.z;
-    const int qb = causal ? P.nqb - 1 - (int)blockIdx.x : (int)blockIdx.x;
-    const int kb0 = 0, kb1 = causal ? qb + 1 : (S + AT_B - 1) / AT_B;
-    const int tid = threadIdx.x, lane = tid & 63;
+    int qb, h, z;
+    if (!prefill_unit(P.nqb, P.H, P.nseq, causal, qb, h, z)) return;
+    const int nkb = P.Sp / AT_B, kb1 = causal ? min(nkb, NQ * (qb + 1)) : nkb;
+    const int tid = threadIdx.x & 255, lane = tid & 63;
+    const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r = lane & 15;
-    const int q0 = qb * AT_B + wave * 16;
-    const size_t kplane = (size_t)P.H * P.Sp * 64;
-    const uint16_t *Kth = P.Kt + ((size_t)z * 2 * P.H + h) * P.Sp * 64;
-    const uint16_t *Vth = P.Vt + ((size_t)z * 3 * P.H + h) * 64 * P.Sp;
-
-    // this lane's query fragments: row q0 + r, dims 32 sl + 8g .. +7, two terms
-    u32x4 aq[2][2];  // [slice][term]
-    {
-        const uint16_t *Qth = P.Qt + ((size_t)z * 2 * P.H + h) * P.Sp * 64 + (size_t)(q0 + r) * 64;
+    const int q0 = (qb * 4 + wave) * 16 * NQ, qa = q0 + r;
+    // group 0: blocks 0, st, 2 st ..; group 1: 1, 1 + st .. (none unsplit)
+    const int st = NG == 2 && kb1 > AT_SPLIT ? 2 : 1, end = st == 1 && grp ? 0 : kb1;
+    // a tile is 40 copies of 1 KiB, ten a wave (past the last block, the last again)
+    const uint16_t *src = P.KV + ((size_t)z * P.H + h) * nkb * AT_TILE;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(&tiles[grp][0][0][0][0]));
+    auto issue = [&](int kb, int stage) {
+        const uint8_t *base = (const uint8_t *)(src + (size_t)(kb < kb1 ? kb : kb1 - 1) * AT_TILE) +
+                              wave * 10240;
+#pragma unroll
+        for (int k = 0; k < 10; ++k)
+            dma16s(base + k * 1024, (uint32_t)lane * 16,
+                   lds0 + stage * (2 * AT_TILE) + wave * 10240 + k * 1024);
+    };
+    if (grp < end) issue(grp, 0);
+    // this lane's query fragments: rows qa + 16 n, dims 32 sl + 8g .. +7, two terms
+    u32x4 aq[NQ][2][2];  // [tile][slice][term]
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+        const int row = min(qa + 16 * n, P.Sp - 1);
+        const uint16_t *Qth = P.Qt + (((size_t)z * 2 * P.H + h) * P.Sp + row) * 64;
 #pragma unroll
         for (int sl = 0; sl < 2; ++sl)
 #pragma unroll
             for (int t = 0; t < 2; ++t)
-                aq[sl][t] = *(const u32x4 *)(Qth + t * (size_t)P.H * P.Sp * 64 + sl * 32 + g * 8);
+                aq[n][sl][t] = *(const u32x4 *)(Qth + t * (size_t)P.H * P.Sp * 64 + sl * 32 + g * 8);
     }
-    float m = -INFINITY, l = 0.0f;  // query q0 + r
-    f32x4 o[4];                      // o[jd][i]: dim 16 jd + 4g + i of query q0 + r
+    float m[NQ], l[NQ];  // query qa + 16 n
+    f32x4 o[NQ][4];      // o[n][jd][i]: dim 16 jd + 4g + i of it
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // staging: 16-byte pieces, 4 of K (term, key, eighth) and 6 of V^T
-    // (term, dim, eighth) per thread; the next key block's pieces are loaded
-    // into registers while the current one is consumed (the last block
-    // reloads itself)
-    u32x4 stg[10];
-    auto load_kv = [&](int kb) {
-        const int k0 = kb * AT_B;
+    for (int n = 0; n < NQ; ++n) {
+        m[n] = -INFINITY;
+        l[n] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int idx = tid + 256 * k, t = idx >> 9, key = (idx >> 3) & 63, pc = idx & 7;
-            stg[k] = *(const u32x4 *)(Kth + t * kplane + (size_t)(k0 + key) * 64 + 8 * pc);
-        }
+        for (int i = 0; i < 4; ++i) o[n][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    int stage = 0;
+    for (int kb = grp; kb - grp < kb1; kb += st) {
+        // the block's copies have landed in every wave, and the other stage's
+        // tile is no longer read
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        __syncthreads();
+        if (kb + st < end) issue(kb + st, stage ^ 1);
+        // (a wave whose queries all lie above the block skips it)
+        if (kb < end && (!causal || kb * AT_B <= q0 + 16 * NQ - 1))
+            prefill_block<NQ>(tiles[grp][stage], aq, kb * AT_B, qa, S, causal, P.scale2, m, l, o);
+        stage ^= 1;
+    }
+    if (NG == 2 && st == 2) {
+        // group 1's state through LDS, [value][thread], merged by group 0
+        __syncthreads();
+        float *x = (float *)&tiles[0][0][0][0][0];
+        if (grp) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            const int idx = tid + 256 * k, t = idx >> 9, dim = (idx >> 3) & 63, pc = idx & 7;
-            stg[4 + k] = *(const u32x4 *)(Vth + t * kplane + (size_t)dim * P.Sp + k0 + 8 * pc);
-        }
-    };
-    const int qa = q0 + r;
-    load_kv(kb0);
-    for (int kb = kb0; kb < kb1; ++kb) {
-        __syncthreads();  // the previous block's K / V are no longer read
+            for (int n = 0; n < NQ; ++n) {
+                x[(18 * n) * 256 + tid] = m[n];
+                x[(18 * n + 1) * 256 + tid] = l[n];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int idx = tid + 256 * k, t = idx >> 9, key = (idx >> 3) & 63, pc = idx & 7;
-            *(u32x4 *)&Ks[t][key][8 * pc] = stg[k];
-        }
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-            const int idx = tid + 256 * k, t = idx >> 9, dim = (idx >> 3) & 63, pc = idx & 7;
-            *(u32x4 *)&Vt[t][dim][8 * pc] = stg[4 + k];
+                for (int e = 0; e < 16; ++e) x[(18 * n + 2 + e) * 256 + tid] = o[n][e >> 2][e & 3];
+            }
         }
         __syncthreads();
-        load_kv(kb + 1 < kb1 ? kb + 1 : kb);
-        __builtin_amdgcn_sched_barrier(0);
-        prefill_block(Ks, Vt, aq, kb * AT_B, qa, S, causal, P.scale, m, l, o);
+        if (grp == 0) {
+#pragma unroll
+            for (int n = 0; n < NQ; ++n) {
+                const float m1 = x[(18 * n) * 256 + tid], l1 = x[(18 * n + 1) * 256 + tid];
+                const float mt = fmaxf(m[n], m1), mref = mt == -INFINITY ? 0.0f : mt;
+                const float a0 = __builtin_amdgcn_exp2f(m[n] - mref);
+                const float a1 = __builtin_amdgcn_exp2f(m1 - mref);
+                l[n] = l[n] * a0 + l1 * a1;
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    o[n][e >> 2][e & 3] =
+                        o[n][e >> 2][e & 3] * a0 + x[(18 * n + 2 + e) * 256 + tid] * a1;
+            }
+        }
     }
-    prefill_store(o, l, qa, S, P.O, P.sout, P.ldo, P.o_vec, h);
+    if (grp == 0)
+#pragma unroll
+        for (int n = 0; n < NQ; ++n)
+            prefill_store(o[n], l[n], qa + 16 * n, S, P.O, P.sout, P.ldo, P.o_vec, h, z);
 }
 
 // The same attention straight from the f32 Q, K and V rows (no term planes
@@ -600,8 +694,8 @@ struct QKVPrefillParams {
     float *O;
     float *kc, *vc;          // KV cache [sequence][head][hs][64], or null
     size_t sin, sout;
-    int S, ld, ldo, causal, nqb, H, hs, rope, o_vec;
-    float scale, rope_step, pos0;
+    int S, ld, ldo, causal, nqb, H, nseq, hs, rope, o_vec;
+    float scale2, rope_step, pos0;
     const float2 *tab;       // (sin, cos) of [row][pair index], or null
 };
 
@@ -615,11 +709,10 @@ __global__ __launch_bounds__(256) void rope_table_kernel(float2 *tab, int S, flo
 }
 
 __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillParams P) {
-    __shared__ __attribute__((aligned(16))) uint16_t Ks[2][AT_B][AT_LD];   // [term][key][dim]
-    __shared__ __attribute__((aligned(16))) uint16_t Vt[3][64][AT_LD];     // [term][dim][key]
+    __shared__ __attribute__((aligned(16))) uint16_t T[5][AT_B][AT_B];  // the key block's tile
     const int S = P.S, causal = P.causal;
-    const int h = blockIdx.y, z = blockIdx.z;
-    const int qb = causal ? P.nqb - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    int qb, h, z;
+    if (!prefill_unit(P.nqb, P.H, P.nseq, causal, qb, h, z)) return;
     const int kb1 = causal ? qb + 1 : P.nqb;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -668,8 +761,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillPara
 
     // the block's raw rows in registers, loaded one block ahead: thread (key
     // kt, quarter kq) holds K dims 8 kq .. +7 and 32 + 8 kq .. +7 with their
-    // rotation angles, and for the V^T items tid and tid + 256 (dim vd, keys
-    // 8 kg .. 8 kg + 7 with kg = tid / 64 + 4 j) the eight V values (each
+    // rotation angles, and for the V^T items tid and tid + 256 (dim vd, piece
+    // kg = tid / 64 + 4 j: keys 32 j + 4 (tid / 64) + i and 16 more) the eight V values (each
     // load instruction reads 64 consecutive dims of one row)
     const int kt = tid >> 2, kq = tid & 3, vd = tid & 63;
     float4 kr[4];
@@ -686,7 +779,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillPara
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const int vrow = min(kb * AT_B + 8 * ((tid >> 6) + 4 * j) + i, S - 1);
+                const int vrow = min(kb * AT_B + 32 * j + 4 * (tid >> 6) + 12 * (i >> 2) + i, S - 1);
                 vv[j][i] = P.V[base + (size_t)vrow * P.ld + vd];
             }
     };
@@ -695,7 +788,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillPara
     // this lane's query fragments: row q0 + r, dims 8g .. +7 and 32 + 8g ..
     // (a RoPE pair per dim), two terms each; zero past the last row
     const int qa = q0 + r;
-    u32x4 aq[2][2];  // [slice][term]
+    u32x4 aq[1][2][2];  // [slice][term]
     {
         const int row = min(qa, S - 1);
         float x1[8], x2[8];
@@ -707,18 +800,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillPara
         if (qa >= S)
 #pragma unroll
             for (int i = 0; i < 8; ++i) x1[i] = x2[i] = 0.0f;
-        split8(x1, aq[0][0], aq[0][1]);
-        split8(x2, aq[1][0], aq[1][1]);
+        split8(x1, aq[0][0][0], aq[0][0][1]);
+        split8(x2, aq[0][1][0], aq[0][1][1]);
     }
-    float m = -INFINITY, l = 0.0f;
-    f32x4 o[4];
+    float m[1] = {-INFINITY}, l[1] = {0.0f};
+    f32x4 o[1][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < 4; ++i) o[0][i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     for (int kb = 0; kb < kb1; ++kb) {
         const int key = kb * AT_B + kt, row = min(key, S - 1);
         const bool ok = key < S, diag = kb == qb && ok;
-        __syncthreads();  // the previous block's Ks and Vt are no longer read
+        __syncthreads();  // the previous block's tile is no longer read
         {
             float x1[8], x2[8];
             unpack8(kr[0], kr[1], x1);
@@ -736,13 +829,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillPara
             }
             u32x4 t0, t1;
             split8(x1, t0, t1);
-            *(u32x4 *)&Ks[0][kt][8 * kq] = t0;
-            *(u32x4 *)&Ks[1][kt][8 * kq] = t1;
+            *(u32x4 *)&T[0][kt][at_piece(kt, kq)] = t0;
+            *(u32x4 *)&T[1][kt][at_piece(kt, kq)] = t1;
             split8(x2, t0, t1);
-            *(u32x4 *)&Ks[0][kt][32 + 8 * kq] = t0;
-            *(u32x4 *)&Ks[1][kt][32 + 8 * kq] = t1;
-            // V^T terms: item (dim vd, key octet kg) splits 8 consecutive keys
-            // (zero past the last row); the diagonal block's raw rows go to
+            *(u32x4 *)&T[0][kt][at_piece(kt, 4 + kq)] = t0;
+            *(u32x4 *)&T[1][kt][at_piece(kt, 4 + kq)] = t1;
+            // V^T terms: item (dim vd, piece kg) splits its 8 keys (zero past
+            // the last row); the diagonal block's raw rows go to
             // the cache, 64 consecutive dims per store instruction
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
@@ -750,24 +843,24 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillPara
                 float x[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    const int vkey = kb * AT_B + 8 * kg + i;
+                    const int vkey = kb * AT_B + 32 * j + 4 * (tid >> 6) + 12 * (i >> 2) + i;
                     x[i] = vkey < S ? vv[j][i] : 0.0f;
                     if (kb == qb && vkey < S && P.vc)
                         P.vc[(((size_t)z * P.H + h) * P.hs + vkey) * 64 + vd] = vv[j][i];
                 }
                 u32x4 t0, t1, t2;
                 split8x3(x, t0, t1, t2);
-                *(u32x4 *)&Vt[0][vd][8 * kg] = t0;
-                *(u32x4 *)&Vt[1][vd][8 * kg] = t1;
-                *(u32x4 *)&Vt[2][vd][8 * kg] = t2;
+                *(u32x4 *)&T[2][vd][at_piece(vd, kg)] = t0;
+                *(u32x4 *)&T[3][vd][at_piece(vd, kg)] = t1;
+                *(u32x4 *)&T[4][vd][at_piece(vd, kg)] = t2;
             }
         }
         __syncthreads();
         if (kb + 1 < kb1) load_kv(kb + 1);
         __builtin_amdgcn_sched_barrier(0);
-        prefill_block(Ks, Vt, aq, kb * AT_B, qa, S, causal, P.scale, m, l, o);
+        prefill_block<1>(T, aq, kb * AT_B, qa, S, causal, P.scale2, m, l, o);
     }
-    prefill_store(o, l, qa, S, P.O, P.sout, P.ldo, P.o_vec, h);
+    prefill_store(o[0], l[0], qa, S, P.O, P.sout, P.ldo, P.o_vec, h, z);
 }
 
 // One launch when the K blocks are rotated by few query blocks and the grid
@@ -812,6 +905,9 @@ int launch_attention_prefill(const float *q, const float *k, const float *v, flo
     VMLM_GUARD(nseq >= 1 && nseq <= 65535 && H <= 65535, "attention prefill: grid too large");
     if (S <= 0) return VMLM_OK;
     const int Sp = (S + AT_B - 1) / AT_B * AT_B;
+    const float scale2 = (float)((double)scale * 1.4426950408889634);
+    VMLM_GUARD((long long)H * nseq <= 1 << 24 && prefill_grid(Sp / AT_B, H * nseq) <= 1 << 30,
+               "attention prefill: grid too large");
     // up to four query blocks over a full grid: one launch from the f32 rows
     // (16-byte rows, no k-slices)
     if (attention_prefill_one_launch(S, H, nseq) && !qs.part && ((uintptr_t)q & 15) == 0 &&
@@ -831,14 +927,15 @@ int launch_attention_prefill(const float *q, const float *k, const float *v, flo
         F.causal = causal ? 1 : 0;
         F.nqb = Sp / AT_B;
         F.H = H;
+        F.nseq = nseq;
         F.hs = hs;
         F.rope = rope ? 1 : 0;
         F.o_vec = ((uintptr_t)out & 15) == 0 && ldo % 4 == 0 && (nseq == 1 || sout % 4 == 0);
-        F.scale = scale;
+        F.scale2 = scale2;
         F.rope_step = rope_step;
         F.pos0 = pos0;
         F.tab = rope && ((uintptr_t)rope_tab & 15) == 0 ? rope_tab : nullptr;  // 16-byte table loads
-        attn_prefill_qkv_kernel<<<dim3(F.nqb, H, nseq), 256, 0, st>>>(F);
+        attn_prefill_qkv_kernel<<<(unsigned)prefill_grid(F.nqb, H * nseq), 256, 0, st>>>(F);
         VMLM_HIP_CHECK(hipGetLastError());
         return VMLM_OK;
     }
@@ -848,8 +945,7 @@ int launch_attention_prefill(const float *q, const float *k, const float *v, flo
     kp.K = k;
     kp.V = v;
     kp.Qt = (uint16_t *)work;
-    kp.Kt = kp.Qt + plane;
-    kp.Vt = kp.Kt + plane;
+    kp.KV = kp.Qt + plane;
     kp.sin = sin;
     kp.S = S;
     kp.Sp = Sp;
@@ -870,19 +966,26 @@ int launch_attention_prefill(const float *q, const float *k, const float *v, flo
     VMLM_HIP_CHECK(hipGetLastError());
     PrefillParams P;
     P.Qt = kp.Qt;
-    P.Kt = kp.Kt;
-    P.Vt = kp.Vt;
+    P.KV = kp.KV;
     P.O = out;
     P.sout = sout;
     P.S = S;
     P.Sp = Sp;
     P.ldo = ldo;
     P.causal = causal ? 1 : 0;
-    P.nqb = Sp / AT_B;
     P.H = H;
     P.o_vec = ((uintptr_t)out & 15) == 0 && ldo % 4 == 0 && (nseq == 1 || sout % 4 == 0);
-    P.scale = scale;
-    attn_prefill_kernel<<<dim3(P.nqb, H, nseq), 256, 0, st>>>(P);
+    P.nseq = nseq;
+    P.scale2 = scale2;
+    // 32 queries a wave once that still gives every CU a workgroup
+    const int nq = (long long)((S + 127) / 128) * H * nseq >= 256 ? 2 : 1;
+    P.nqb = (S + 64 * nq - 1) / (64 * nq);
+    const unsigned grid = (unsigned)prefill_grid(P.nqb, H * nseq);
+    const bool one = Sp / AT_B <= AT_SPLIT;  // no query block is split: one group
+    if (nq == 2 && one) attn_prefill_kernel<2, 1><<<grid, 256, 0, st>>>(P);
+    else if (nq == 2) attn_prefill_kernel<2, 2><<<grid, 512, 0, st>>>(P);
+    else if (one) attn_prefill_kernel<1, 1><<<grid, 256, 0, st>>>(P);
+    else attn_prefill_kernel<1, 2><<<grid, 512, 0, st>>>(P);
     VMLM_HIP_CHECK(hipGetLastError());
     return VMLM_OK;
 }

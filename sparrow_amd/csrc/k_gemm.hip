@@ -55,40 +55,6 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// s_waitcnt immediate (gfx9 encoding) that waits for the vector-memory
-// counter to drop to n and leaves the other counters unconstrained.
-constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 4) | (0xF << 8); }
-
-// One 16-byte-per-lane copy from global memory into LDS: lane i's 16 bytes
-// at gptr land at LDS byte address lds_base + 16 * i (lds_base wave-uniform).
-// Issued as inline assembly so that the compiler does not order every later
-// LDS read behind it; the callers wait for the copies with explicit vmcnt
-// waits and publish them with barriers. m0 is not used by anything else in
-// these kernels.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved; nothing else here uses it
-__device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(gptr), "s"(lds_base)
-                 : "memory", "m0");
-}
-
-// The same copy with a wave-uniform base held in SGPRs (sbase) and a 32-bit
-// per-lane byte offset: one VGPR per distinct offset instead of a 64-bit
-// address per copy.
-__device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(lds_base)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-__device__ __forceinline__ uint32_t lds_addr(const void *p) {
-    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)p;
-}
-
 // 8 int8 weights -> 8 bf16 (exact).
 __device__ __forceinline__ u32x4 i8x8_to_bf16(uint32_t w0, uint32_t w1) {
     uint32_t d[4];

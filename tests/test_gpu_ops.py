@@ -454,6 +454,20 @@ def test_attention_prefill(ops, oracle, S, H):
     assert np.array_equal(got[0], v[0]) or np.abs(got[0] - v[0]).max() <= 1e-6
 
 
+# Rows at the edges of the 64-key blocks and of the 64- and 128-query blocks, up
+# to four key blocks (one group of waves) and past them (two groups merged, odd
+# and even block counts), with (sequence, head) counts dealt to the XCDs (8,
+# 36) and not (2, 12), with and without the causal mask.
+@pytest.mark.parametrize("S,H,causal", [(1, 2, True), (64, 8, False), (65, 36, True),
+                                        (256, 2, True), (257, 12, True), (320, 8, False),
+                                        (385, 2, True), (449, 36, True), (600, 36, False)])
+def test_attention_prefill_blocks(ops, oracle, S, H, causal):
+    rng = np.random.default_rng(S + H)
+    q, k, v = (rng.standard_normal((S, H * 64), dtype=np.float32) for _ in range(3))
+    got = ops.attention_prefill(q, k, v, H, pos0=3, causal=causal)
+    assert_close_rms(got, oracle.attention_prefill(q, k, v, H, pos0=3, causal=causal))
+
+
 def test_attention_prefill_one_launch_same_bits(ops, oracle):
     """Up to four 64-query blocks (S <= 256) over at least 256 workgroups
     (query blocks x heads) run as one launch from the f32 rows; longer
