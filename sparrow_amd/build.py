@@ -27,10 +27,10 @@ COMMON = [
 ]
 
 
-# Per-file flags. k_gemm.hip, k_direct.hip: MFMA accumulators in arch VGPRs rather than
+# Per-file flags. k_gemm.hip, k_gemm32.hip, k_direct.hip: MFMA accumulators in arch VGPRs rather than
 # AGPRs (the 16 x 16 products issue at about half rate with AGPR
 # accumulators on gfx950; config 1's bf16 GEMM 5.73 -> 5.42 us)
-EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("k_gemm.hip", "k_direct.hip")}
+EXTRA = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("k_gemm.hip", "k_gemm32.hip", "k_direct.hip")}
 
 
 def _compile(src: Path) -> Path:

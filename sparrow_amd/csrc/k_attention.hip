@@ -21,156 +21,6 @@
 
 namespace vmlm {
 
-// ---------------------------------------------------------------- f32 GEMM
-// C[m,n] (+)= A[m,k] . op(B), op(B) = B[n,k]^T (nt) or B[k,n], on the f32
-// matrix cores: v_mfma_f32_16x16x4f32 multiplies f32 operands exactly and
-// accumulates in f32 (only the summation order differs from the reference's
-// FMA chains, inside the 1e-4 * RMS contract of the attention composition).
-// 32 x 32 tiles, four waves of 16 x 16 (lane (g, r) = (lane / 16, lane % 16)
-// gives A[row r][k g] and op(B)[k g][col r] and holds rows 4g..4g+3 of column
-// r). 64-deep k-steps through LDS: A as [row][k], an NT B as [col][k], an NN
-// B as [k][col]; the next step's tiles are loaded into registers while the
-// current one is consumed. With VEC the rows are read as float4 (k, or n for
-// an NN B, a multiple of 4 and 16-byte aligned operands). A grid of few tiles
-// is split over k (grid z): each slice writes its partial tile to `part`
-// [ks][m][n] and gemm_f32_reduce_kernel sums the slices in order
-// (deterministic).
-constexpr int GF_T = 32, GF_K = 64;
-constexpr int GF_LDA = GF_K + 4;   // [row][k] pitch (floats)
-constexpr int GF_LDB = GF_T + 16;  // [k][col] pitch: lanes (g, r) two-way at most
-
-template <bool NT, bool VEC>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float *__restrict__ A,
-                                                       const float *__restrict__ B,
-                                                       float *__restrict__ C, int m, int n, int k,
-                                                       int acc, int kslice,
-                                                       float *__restrict__ part) {
-    __shared__ __attribute__((aligned(16))) float As[GF_T][GF_LDA];
-    __shared__ __attribute__((aligned(16))) float Bs[NT ? GF_T : GF_K][NT ? GF_LDA : GF_LDB];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1, g = lane >> 4, r = lane & 15;
-    const int row0 = blockIdx.y * GF_T, col0 = blockIdx.x * GF_T;
-    const int kb = blockIdx.z * kslice;
-    const int ke = kb + kslice < k ? kb + kslice : k;
-    auto ld4 = [&](const float *p, bool ok, int left) {
-        if constexpr (VEC) {
-            return ok && left >= 4 ? *(const float4 *)p : make_float4(0.f, 0.f, 0.f, 0.f);
-        } else {
-            return make_float4(ok && left > 0 ? p[0] : 0.f, ok && left > 1 ? p[1] : 0.f,
-                               ok && left > 2 ? p[2] : 0.f, ok && left > 3 ? p[3] : 0.f);
-        }
-    };
-    // loader roles (two float4 per thread and operand): A and an NT B as 32
-    // rows x 16 float4 of k; an NN B as 64 k-rows x 8 float4 of n
-    float4 ra[2], rb[2];
-    auto load = [&](int k0) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int e = tid + q * 256, rr = e >> 4, c4 = (e & 15) * 4, gk = k0 + c4;
-            const int gr = row0 + rr;
-            ra[q] = ld4(A + (size_t)(gr < m ? gr : 0) * k + (gk < ke ? gk : kb), gr < m, ke - gk);
-            if constexpr (NT) {
-                const int gc = col0 + rr;
-                rb[q] = ld4(B + (size_t)(gc < n ? gc : 0) * k + (gk < ke ? gk : kb), gc < n, ke - gk);
-            } else {
-                const int kr = e >> 3, n4 = (e & 7) * 4, gkr = k0 + kr, gc = col0 + n4;
-                rb[q] = ld4(B + (size_t)(gkr < ke ? gkr : kb) * n + (gc < n ? gc : 0), gkr < ke,
-                            n - gc);
-            }
-        }
-    };
-    auto store = [&]() {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int e = tid + q * 256, rr = e >> 4, c4 = (e & 15) * 4;
-            *(float4 *)&As[rr][c4] = ra[q];
-            if constexpr (NT) *(float4 *)&Bs[rr][c4] = rb[q];
-            else *(float4 *)&Bs[e >> 3][(e & 7) * 4] = rb[q];
-        }
-    };
-    f32x4 d = {0.f, 0.f, 0.f, 0.f};
-    load(kb);
-    for (int k0 = kb; k0 < ke; k0 += GF_K) {
-        __syncthreads();
-        store();
-        __syncthreads();
-        if (k0 + GF_K < ke) load(k0 + GF_K);
-#pragma unroll
-        for (int kk = 0; kk < GF_K; kk += 4) {
-            const float a = As[wm * 16 + r][kk + g];
-            const float b = NT ? Bs[wn * 16 + r][kk + g] : Bs[kk + g][wn * 16 + r];
-            d = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, d, 0, 0, 0);
-        }
-    }
-    const int gc = col0 + wn * 16 + r;
-    if (gc >= n) return;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int gr = row0 + wm * 16 + 4 * g + q;
-        if (gr >= m) continue;
-        if (part) {
-            part[((size_t)blockIdx.z * m + gr) * n + gc] = d[q];
-        } else {
-            float *o = C + (size_t)gr * n + gc;
-            *o = acc ? *o + d[q] : d[q];
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const float *__restrict__ part,
-                                                              int ks, size_t mn,
-                                                              float *__restrict__ C, int acc) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= mn) return;
-    float v = part[i];
-    for (int z = 1; z < ks; ++z) v += part[(size_t)z * mn + i];
-    C[i] = acc ? C[i] + v : v;
-}
-
-size_t gemm_f32_work_floats(size_t m, size_t n, size_t k) {
-    const size_t tiles = cdiv(m, (size_t)GF_T) * cdiv(n, (size_t)GF_T);
-    if (tiles >= 128 || k < 2 * GF_K) return 0;
-    size_t ks = cdiv((size_t)256, tiles);
-    const size_t steps = cdiv(k, (size_t)GF_K);
-    ks = ks < steps ? ks : steps;
-    return ks > 1 ? ks * m * n : 0;
-}
-
-int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n, size_t k,
-                    bool acc, bool b_is_nt, hipStream_t st, float *work) {
-    if (m == 0 || n == 0) return VMLM_OK;
-    if (k == 0) {
-        if (!acc) return launch_fill_zero(c, m * n * sizeof(float), st);
-        return VMLM_OK;
-    }
-    VMLM_GUARD(m <= 0x7fffffffu && n <= 0x7fffffffu && k <= 0x7fffffffu, "gemm f32: shape too large");
-    // split k when the output is narrow (and the caller gave the workspace)
-    const size_t wf = gemm_f32_work_floats(m, n, k);
-    int ks = 1;
-    if (wf && work) ks = (int)(wf / (m * n));
-    const size_t steps = cdiv(k, (size_t)GF_K);
-    const int kslice = (int)(cdiv(steps, (size_t)ks) * GF_K);
-    ks = (int)cdiv(k, (size_t)kslice);
-    const bool vec = k % 4 == 0 && (b_is_nt || n % 4 == 0) && ((uintptr_t)a & 15) == 0 &&
-                     ((uintptr_t)b & 15) == 0;
-    float *part = ks > 1 ? work : nullptr;
-    dim3 grid(cdiv(n, (size_t)GF_T), cdiv(m, (size_t)GF_T), ks);
-    const int ia = acc ? 1 : 0, ik = (int)k;
-    if (b_is_nt) {
-        if (vec) gemm_f32_kernel<true, true><<<grid, 256, 0, st>>>(a, b, c, (int)m, (int)n, ik, ia, kslice, part);
-        else gemm_f32_kernel<true, false><<<grid, 256, 0, st>>>(a, b, c, (int)m, (int)n, ik, ia, kslice, part);
-    } else {
-        if (vec) gemm_f32_kernel<false, true><<<grid, 256, 0, st>>>(a, b, c, (int)m, (int)n, ik, ia, kslice, part);
-        else gemm_f32_kernel<false, false><<<grid, 256, 0, st>>>(a, b, c, (int)m, (int)n, ik, ia, kslice, part);
-    }
-    VMLM_HIP_CHECK(hipGetLastError());
-    if (part) {
-        gemm_f32_reduce_kernel<<<cdiv(m * n, (size_t)256), 256, 0, st>>>(part, ks, m * n, c, ia);
-        VMLM_HIP_CHECK(hipGetLastError());
-    }
-    return VMLM_OK;
-}
-
 // ---------------------------------------------------------------- prefill
 // Q, K already rotated; all [S][ld] with head h at columns h*64.
 //

@@ -1,0 +1,345 @@
+// k_gemm32.hip -- f32 GEMM on the f32 matrix cores.
+//
+// C[m,n] (+)= A[m,k] . op(B), op(B) = B[n,k]^T (NT: gemm_nt,
+// ops/src/kernels.rs:986-1015) or B[k,n] (NN: gemm, :406-419).
+// v_mfma_f32_16x16x4f32 multiplies f32 operands exactly and accumulates in f32
+// (only the summation order differs from the reference's FMA chains, inside the
+// 1e-4 * RMS contract of the attention composition).
+//
+// BM x BN tiles, four waves of 2 x 2. 32- or 64-deep k-steps go straight from
+// global memory into a two-stage LDS ring, the next step's copies in flight while
+// one is multiplied (three stages, so fewer workgroups a CU, were 1 to 4 %
+// slower), or, where the rows are not 16-byte aligned, through registers. An
+// operand stored along k ([row][k]) keeps its 16-byte
+// pieces swizzled by row against bank conflicts, and a lane
+// (g, r) = (lane / 16, lane % 16) reads four consecutive k of row r, one for each
+// of four MFMAs (MFMA e of a 16-deep group multiplies k = 4g + e: any assignment
+// that both operands share gives the same products). An NN B ([k][col]) keeps
+// piece c of row k in slot c ^ 4 (k / 4 % 4), so that the four groups' rows meet
+// other banks. Elements past k are copied from a zero; rows and columns past m
+// and n repeat the last and are not stored.
+//
+// The MFMA rate bounds large shapes (a 16 x 16 x 4 product takes a matrix core 32
+// cycles; the clock settles near 2.1 GHz under them), so the tile is chosen for an
+// even load of the CUs. Against a register-staged kernel of 32 x 32 tiles: 1000 x
+// 2304 x 2304 NT 125 -> 113 us, 2048^3 176 -> 140 (123 TFLOP/s), 4096^3 1400 ->
+// 1045, 1500 x 1537 x 1535 (rows off 16 bytes) 193 -> 88. A rotated order of the
+// steps per tile (to spread the L2 channels of rows 9 KiB apart) changed nothing. A grid of few tiles
+// is split over k (grid z): each slice writes its partial tile to `part`
+// [ks][m][n] and gemm_f32_reduce_kernel sums the slices in order (deterministic).
+#include "internal.hpp"
+
+namespace vmlm {
+
+namespace {
+
+// k of a step: 64 for the smallest tile (its 32-deep steps are mostly barriers)
+template <int BM, int BN>
+constexpr int g32_k() {
+    return BM == 32 && BN == 32 ? 64 : 32;
+}
+
+__device__ __attribute__((aligned(16))) float g32_zero[4];
+
+typedef f32x4 f32x4_w __attribute__((aligned(4)));
+
+// LDS row of an NN B's k-row (and back): 32 columns are half of the banks, so
+// groups 2 and 3 of a 16-deep group take the row of the other half.
+template <int BN>
+__device__ __forceinline__ int nn_row(int k) {
+    return BN == 32 ? k ^ ((k >> 3) & 1) : k;
+}
+
+struct G32Params {
+    const float *A, *B;
+    float *C, *part;
+    int m, n, k, acc, kslice, group;
+};
+
+template <bool NT, bool VEC, int BM, int BN>
+__global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
+    constexpr int KS = g32_k<BM, BN>(), ROW = KS * 4, PK = KS / 4;  // pieces of a row along k
+    constexpr int A_BYTES = BM * ROW, B_BYTES = BN * ROW, STAGE = A_BYTES + B_BYTES;
+    constexpr int A_INS = A_BYTES / 4096, B_INS = B_BYTES / 4096;  // pieces a lane copies a step
+    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
+    static_assert(A_INS >= 1 && B_INS >= 1 && TM >= 1 && TN >= 1, "tile too small");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * STAGE];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1, g = lane >> 4, r = lane & 15;
+    int tbx, tby;
+    gemm_tile(p.group, tbx, tby);
+    const int m0 = tby * BM, n0 = tbx * BN;
+    const int kb = (int)blockIdx.z * p.kslice;
+    const int ke = kb + p.kslice < p.k ? kb + p.kslice : p.k;
+    const int nk = (ke - kb + KS - 1) / KS;
+    // slot of piece c of row R (rows along k): 128-byte rows share the banks in
+    // pairs, 256-byte rows each hold all of them
+    auto slot = [](int R, int c) { return c ^ (KS == 32 ? (R >> 1) & 7 : R & 15); };
+
+    // this lane's source of each copy at step 0, and its k within the step
+    const float *as[A_INS], *bs[B_INS];
+    int ak[A_INS], bk[B_INS], bn[B_INS];
+#pragma unroll
+    for (int q = 0; q < A_INS; ++q) {
+        const int off = ((q * 4 + wave) * 64 + lane) * 16, R = off / ROW;
+        ak[q] = slot(R, (off >> 4) & (PK - 1)) * 4;
+        const int row = m0 + R;
+        as[q] = p.A + (size_t)(row < p.m ? row : p.m - 1) * p.k + kb + ak[q];
+    }
+#pragma unroll
+    for (int q = 0; q < B_INS; ++q) {
+        const int off = ((q * 4 + wave) * 64 + lane) * 16;
+        if constexpr (NT) {
+            const int R = off / ROW;
+            bk[q] = slot(R, (off >> 4) & (PK - 1)) * 4;
+            bn[q] = 4;
+            const int row = n0 + R;
+            bs[q] = p.B + (size_t)(row < p.n ? row : p.n - 1) * p.k + kb + bk[q];
+        } else {
+            constexpr int PPR = BN / 4;  // pieces per k-row
+            bk[q] = nn_row<BN>(off / (BN * 4));
+            const int c = ((off >> 4) & (PPR - 1)) ^ ((4 * (bk[q] >> 2)) & (PPR - 1) & 12);
+            // (columns past n: a piece of the row's start, not stored)
+            bn[q] = p.n - (n0 + 4 * c);
+            const int col = bn[q] > 0 ? n0 + 4 * c : 0;
+            bs[q] = p.B + (size_t)(kb + bk[q]) * p.n + col;
+        }
+    }
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(smem));
+    const size_t bstep = NT ? KS : (size_t)KS * p.n;
+    auto issue = [&](int kt) {  // rows of whole 16-byte pieces, straight into LDS
+        const uint32_t sb = lds0 + (uint32_t)((kt & 1) * STAGE);
+        const bool tail = kb + (kt + 1) * KS > ke;
+        auto copy = [&](const float *src, int kin, uint32_t dst) {
+            if (tail && kb + kt * KS + kin >= ke) src = g32_zero;
+            dma16(src, dst);
+        };
+#pragma unroll
+        for (int q = 0; q < A_INS; ++q) copy(as[q] + kt * KS, ak[q], sb + (q * 4 + wave) * 1024);
+#pragma unroll
+        for (int q = 0; q < B_INS; ++q)
+            copy(bs[q] + kt * bstep, bk[q], sb + A_BYTES + (q * 4 + wave) * 1024);
+    };
+    // rows at any float: the pieces through registers, those that cross the end
+    // of a row (the last step, an NN B's last columns) element by element
+    f32x4 ra[A_INS], rb[B_INS];
+    auto load = [&](int kt) {
+        const int left = ke - (kb + kt * KS);
+        const bool whole = left >= KS && (NT || n0 + BN <= p.n);
+        auto piece = [&](const float *src, int valid) {
+            f32x4 v = {0.f, 0.f, 0.f, 0.f};
+            if (valid >= 4) v = *(const f32x4_w *)src;
+            else
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e < valid) v[e] = src[e];
+            return v;
+        };
+#pragma unroll
+        for (int q = 0; q < A_INS; ++q) {
+            const float *src = as[q] + kt * KS;
+            ra[q] = left >= KS ? *(const f32x4_w *)src : piece(src, left - ak[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < B_INS; ++q) {
+            const float *src = bs[q] + kt * bstep;
+            rb[q] = whole ? *(const f32x4_w *)src
+                    : NT  ? piece(src, left - bk[q])
+                          : piece(src, bk[q] < left ? bn[q] : 0);
+        }
+    };
+    auto store = [&](int kt) {
+        uint8_t *sb = smem + (kt & 1) * STAGE + (wave * 64 + lane) * 16;
+#pragma unroll
+        for (int q = 0; q < A_INS; ++q) *(f32x4 *)(sb + q * 4096) = ra[q];
+#pragma unroll
+        for (int q = 0; q < B_INS; ++q) *(f32x4 *)(sb + A_BYTES + q * 4096) = rb[q];
+    };
+
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const uint8_t *sA) {
+        const uint8_t *sB = sA + A_BYTES;
+#pragma unroll
+        for (int h = 0; h < KS / 16; ++h) {
+            const int at = slot(r, 4 * h + g) * 16;  // rows 16 i + r alike
+            f32x4 a[TM], b[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                a[i] = *(const f32x4 *)(sA + (wm * WM + 16 * i + r) * ROW + at);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int col = wn * WN + 16 * j + r;
+                if constexpr (NT) {
+                    b[j] = *(const f32x4 *)(sB + col * ROW + at);
+                } else {
+                    const int cs = (col >> 2) ^ ((4 * g) & (BN / 4 - 1) & 12);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        b[j][e] = *(const float *)(sB + nn_row<BN>(16 * h + 4 * g + e) * (BN * 4) +
+                                                   cs * 16 + (col & 3) * 4);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e],
+                                                                         acc[i][j], 0, 0, 0);
+        }
+    };
+    if constexpr (VEC) issue(0);
+    else load(0);
+    for (int kt = 0; kt < nk; ++kt) {
+        // step kt is in LDS, and every wave has read step kt - 1
+        if constexpr (VEC) __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        else store(kt);
+        __syncthreads();
+        if (kt + 1 < nk) {
+            if constexpr (VEC) issue(kt + 1);
+            else load(kt + 1);
+        }
+        compute(smem + (kt & 1) * STAGE);
+    }
+
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int col = n0 + wn * WN + 16 * j + r;
+            if (col >= p.n) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = m0 + wm * WM + 16 * i + 4 * g + e;
+                if (row >= p.m) continue;
+                if (p.part) {
+                    p.part[((size_t)blockIdx.z * p.m + row) * p.n + col] = acc[i][j][e];
+                } else {
+                    float *o = p.C + (size_t)row * p.n + col;
+                    *o = p.acc ? *o + acc[i][j][e] : acc[i][j][e];
+                }
+            }
+        }
+}
+
+constexpr int G32_SLICES = 16;
+__global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const float *__restrict__ part,
+                                                              int ks, size_t mn,
+                                                              float *__restrict__ C, int acc) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= mn) return;
+    float v[G32_SLICES];  // every slice in flight, then summed in order
+#pragma unroll
+    for (int z = 0; z < G32_SLICES; ++z) v[z] = part[(size_t)(z < ks ? z : ks - 1) * mn + i];
+    float sum = v[0];
+#pragma unroll
+    for (int z = 1; z < G32_SLICES; ++z)
+        if (z < ks) sum += v[z];
+    C[i] = acc ? C[i] + sum : sum;
+}
+
+// The tile with the least work on the busiest CU: `f` weighs what a smaller tile
+// copies per product (128 x 128: 129 TFLOP/s at 4096^3; 64 x 64 119, 32 x 64 107,
+// 32 x 32 102), `one` what it loses alone on its CU (fewer accumulators to keep
+// a matrix core busy). Then the k-slices, of 128 at least, that give a small
+// grid about two workgroups per CU (the second launch costs about five steps).
+struct Shape {
+    int bm, bn, ks;
+};
+Shape pick_tile(size_t m, size_t n) {
+    struct Tile {
+        int bm, bn;
+        double f, one;
+    };
+    constexpr Tile tiles[] = {{128, 128, 1.0, 1.0}, {64, 64, 1.08, 1.1}, {32, 64, 1.17, 1.15},
+                              {32, 32, 1.26, 1.0}};
+    Shape best{32, 32, 1};
+    if ((size_t)cdiv(m, 32) * cdiv(n, 32) <= 256) return best;  // one round of the smallest
+    double least = 1e300;
+    for (const Tile &t : tiles) {
+        const size_t wgs = (size_t)cdiv(m, t.bm) * cdiv(n, t.bn), per = (wgs + 255) / 256;
+        const double load = (double)per * t.bm * t.bn * t.f * (per == 1 ? t.one : 1.0);
+        if (load < least) {
+            least = load;
+            best.bm = t.bm;
+            best.bn = t.bn;
+        }
+    }
+    return best;
+}
+Shape pick_shape(size_t m, size_t n, size_t k) {
+    Shape best = pick_tile(m, n);
+    const size_t wgs = (size_t)cdiv(m, best.bm) * cdiv(n, best.bn), steps = (k + 63) / 64;
+    if (wgs <= 128 && steps >= 8) {
+        size_t ks = 512 / wgs;
+        if (ks > steps / 2) ks = steps / 2;
+        if (ks > G32_SLICES) ks = G32_SLICES;
+        best.ks = (int)ks;
+    }
+    return best;
+}
+
+template <bool NT, bool VEC, int BM, int BN>
+int launch_tile(const G32Params &p, int ks, hipStream_t st) {
+    const dim3 grid(cdiv((size_t)p.n, BN), cdiv((size_t)p.m, BM), ks);
+    gemm_f32_kernel<NT, VEC, BM, BN><<<grid, 256, 0, st>>>(p);
+    VMLM_HIP_CHECK(hipGetLastError());
+    return VMLM_OK;
+}
+template <bool NT, bool VEC>
+int launch_shape(const G32Params &p, const Shape &s, hipStream_t st) {
+    if (s.bm == 128) return launch_tile<NT, VEC, 128, 128>(p, s.ks, st);
+    if (s.bm == 64) return launch_tile<NT, VEC, 64, 64>(p, s.ks, st);
+    if (s.bn == 64) return launch_tile<NT, VEC, 32, 64>(p, s.ks, st);
+    return launch_tile<NT, VEC, 32, 32>(p, s.ks, st);
+}
+
+}  // namespace
+
+size_t gemm_f32_work_floats(size_t m, size_t n, size_t k) {
+    const int ks = pick_shape(m, n, k).ks;
+    return ks > 1 ? (size_t)ks * m * n : 0;
+}
+
+int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n, size_t k,
+                    bool acc, bool b_is_nt, hipStream_t st, float *work) {
+    if (m == 0 || n == 0) return VMLM_OK;
+    if (k == 0) {
+        if (!acc) return launch_fill_zero(c, m * n * sizeof(float), st);
+        return VMLM_OK;
+    }
+    VMLM_GUARD(m <= 0x7fffffffu && n <= 0x7fffffffu && k <= 0x7fffffc0u,
+               "gemm f32: shape too large");
+    Shape s = pick_shape(m, n, k);
+    if (!work) s.ks = 1;
+    const size_t steps = (k + 63) / 64;
+    G32Params p;
+    p.A = a;
+    p.B = b;
+    p.C = c;
+    p.m = (int)m;
+    p.n = (int)n;
+    p.k = (int)k;
+    p.acc = acc ? 1 : 0;
+    p.kslice = (int)((steps + s.ks - 1) / s.ks * 64);
+    s.ks = (int)((k + p.kslice - 1) / p.kslice);
+    p.part = s.ks > 1 ? work : nullptr;
+    p.group = s.ks > 1 ? 0 : 8;
+    const bool vec = k % 4 == 0 && (b_is_nt || n % 4 == 0) && ((uintptr_t)a & 15) == 0 &&
+                     ((uintptr_t)b & 15) == 0;
+    const int rc = b_is_nt ? vec ? launch_shape<true, true>(p, s, st) : launch_shape<true, false>(p, s, st)
+                           : vec ? launch_shape<false, true>(p, s, st) : launch_shape<false, false>(p, s, st);
+    if (rc || !p.part) return rc;
+    gemm_f32_reduce_kernel<<<cdiv(m * n, (size_t)256), 256, 0, st>>>(work, s.ks, m * n, c, p.acc);
+    VMLM_HIP_CHECK(hipGetLastError());
+    return VMLM_OK;
+}
+
+}  // namespace vmlm

@@ -245,3 +245,32 @@ def test_gemm_direct_infinite_and_nan_rows(dev):
         assert np.array_equal(f(got), f(ref))
     ok = np.isfinite(ref)
     assert np.abs(got[ok] - ref[ok]).max() <= 1e-5 * np.sqrt(np.mean(ref[ok] ** 2))
+
+
+# f32 GEMM: each tile (32 x 32, 32 x 64, 64 x 64, 128 x 128), rows and columns at
+# their edges, k at the 32-deep steps' edges, rows on and off 16 bytes (k % 4, n %
+# 4, operands a float off), with k-slices and without, NT and NN.
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 33, 31), (33, 2305, 96), (40, 100, 1030),
+                                   (513, 1028, 64), (1030, 1020, 36), (2049, 2052, 33)])
+def test_gemm_f32_edges(dev, m, n, k):
+    """Against float64: at most ceil(k / 16) chains of four products in one
+    accumulator, then up to 16 slices: (k + 20) roundings of 2^-24 of
+    sum |a b|."""
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((n, k), dtype=np.float32)
+    c0 = rng.standard_normal((m, n), dtype=np.float32)
+    ref = a.astype(np.float64) @ b.astype(np.float64).T
+    bound = (k + 20) * 2.0 ** -24 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T +
+                                     np.abs(c0))
+    zero = np.zeros(1, np.float32)
+    for off in (0, 1):
+        pad = zero[:off]
+        da = C.c_void_p(dev.up(np.concatenate([pad, a.ravel()])).value + 4 * off)
+        for f, bb in ((dev.lib.vmlm_hip_gemm_nt, b), (dev.lib.vmlm_hip_gemm, b.T)):
+            db = C.c_void_p(dev.up(np.concatenate([pad, bb.ravel()])).value + 4 * off)
+            for acc in (False, True):
+                dc = dev.up(c0)
+                dev.check(f(da, db, dc, m, n, k, acc, None))
+                got = dev.down(dc, (m, n), np.float32).astype(np.float64)
+                assert (np.abs(got - (ref + c0 if acc else ref)) <= bound).all()
