@@ -560,7 +560,10 @@ int vmlm_hip_memcpy_d2d(void *dst, const void *src, size_t bytes) {
 }
 int vmlm_hip_memset(void *dptr, int value, size_t bytes) {
     INIT_OR_RETURN();
+    // hipMemset may return before the memory is set, and it runs on the legacy
+    // stream, which the library's non-blocking stream does not wait for
     VMLM_HIP_CHECK(hipMemset(dptr, value, bytes));
+    VMLM_HIP_CHECK(hipStreamSynchronize(nullptr));
     return VMLM_OK;
 }
 
