@@ -271,9 +271,8 @@ static inline size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; 
 //    direct kernel only takes its small grids (1 x 2304 x 2304: 7.3 -> 6.3,
 //    equal near 20 us); with more rows it reads the activation again for every
 //    16 columns (16 x 122753 x 2304: 294 -> 108, 16 x 2304 x 2304: 14.3 -> 6.9);
-//  * unpadded int8 at m > 16: int8 rows, the GEMM, the slice reduction and the
-//    non-finite rows are four launches, 9 + 0.2 per k-step and the products
-//    at 500 TFLOP/s (17 x 2304 x 2304: 17.0 -> 7.2; 64 x 5760 x 2304: 21.1 ->
+//  * unpadded int8 at m > 16: int8 rows, the GEMM and the slice reduction are
+//    three launches, 7 + 0.2 per k-step and the products at 500 TFLOP/s (17 x 2304 x 2304: 17.0 -> 7.2; 64 x 5760 x 2304: 21.1 ->
 //    15.8; 100 x 2304 x 5760: 27.6 -> 20.5); up to 128 rows, above which the
 //    row blocks of the int8 GEMM are full (300 x 5760 x 2304: 39 against 44);
 //  * else the padded weight copy, the term planes and the bf16 GEMM: 10, the
@@ -285,7 +284,7 @@ static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
     if (k == 0 || m > 4096 || n > (size_t)1 << 24 || k > (size_t)1 << 24) return false;
     const double us = gemm_direct_us((int)m, (int)n, (int)k, wi8);
     const double nk = (double)((k + 63) / 64), flop = 2.0 * m * n * k;
-    if (!padded && wi8) return m > 16 && m <= 128 && us < 9.0 + 0.2 * nk + flop / 500e6;
+    if (!padded && wi8) return m > 16 && m <= 128 && us < 7.0 + 0.2 * nk + flop / 500e6;
     if (!padded && m <= 16) return m > 5 || us < 20.0;
     const double steps = 1.2 * nk, prod = flop / 230e6;
     const double copy = padded ? 2.0 * n * k * (wi8 ? 1 : 2) / 4e6 : 0.0;
@@ -420,10 +419,14 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
         const size_t gw = gemm_i8_work_floats((int)m, (int)n, (int)k);
         float *gwork = gw ? stg.template alloc<float>(gw) : nullptr;
         // many rows: the weights swizzled into 1 KiB blocks first (one pass
-        // over N x K bytes), so the GEMM's weight copies move whole blocks;
-        // the allocation-free entry point keeps its scratch for the rows
-        // (a swizzled copy the caller keeps is read as it is)
-        const bool blk = Wsw || (std::is_same<WS, Stage>::value && m >= 256 && n % 16 == 0);
+        // over N x K bytes), so the GEMM's weight copies move whole blocks,
+        // where the GEMM is long enough to pay for the pass (K = 2304: 512 x
+        // 2304 36.5 with it, 31.8 without, 1500 x 2304 49.5 and 48.3, 2048 x
+        // 11520 177 and 186; 700 x 2304 x 5760 59.7 and 62.2); the
+        // allocation-free entry point keeps its scratch for the rows (a
+        // swizzled copy the caller keeps is read as it is)
+        const bool blk = Wsw || (std::is_same<WS, Stage>::value && m >= 256 &&
+                                 m * k >= (size_t)3600000 && n % 16 == 0);
         int8_t *wsw = blk && !Wsw ? stg.template alloc<int8_t>(n * k) : nullptr;
         STAGE_OK(stg);
         int rc = launch_rows_q8(a, k, nullptr, 0.0f, m, k, a8, a8s, st);
@@ -432,6 +435,10 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
         GemmArgs g;
         g.W = Wsw ? Wsw : blk ? (const void *)wsw : Wd;
         g.w_blocked = blk;
+        g.nf.f = a8s;
+        g.nf.x = a;
+        g.nf.q = (const int8_t *)Wd;
+        g.nf.ldx = g.nf.ldq = g.nf.K = (int)k;
         g.w_int8 = true;
         g.scale = scale;
         g.A8 = a8;
@@ -444,10 +451,7 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
         g.K = (int)k;
         g.C = c;
         g.ldc = (int)n;
-        rc = launch_gemm(g, st);
-        if (rc) return rc;
-        return launch_gemm_i8_nonfinite_rows(a, (int)k, (const int8_t *)Wd, (int)k, scale, a8s, c,
-                                             (int)n, (int)m, (int)n, (int)k, st);
+        return launch_gemm(g, st);
     }
     uint16_t *terms = stg.template alloc<uint16_t>((size_t)T * m * Kp);
     STAGE_OK(stg);

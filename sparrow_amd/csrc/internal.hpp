@@ -84,9 +84,40 @@ struct GemvArgs {
     int ldx = 0;
 };
 int launch_gemv(const GemvArgs &a, hipStream_t st);
-// C = (in-order sum of ks k-slice partials [ks][M][N]) * scale (per column, or none).
+// The rows of an int8-row GEMM that hold a NaN or an infinity (their factor is
+// NaN, q8_row_k): the kernel that writes C recomputes their elements from the
+// f32 rows and the row-major int8 weights (nonfinite_dot).
+struct NonfiniteRows {
+    const float *f = nullptr;  // row factors [M]
+    const float *x = nullptr;  // f32 rows
+    const int8_t *q = nullptr;  // weights [N][ldq]
+    int ldx = 0, ldq = 0, K = 0;
+};
+
+// x[row] . q[col] in the reference's order (ops/src/kernels.rs:1256-1287: eight
+// FMA lanes over k, the 8 -> 1 fold, the scalar tail), so the +-inf / NaN
+// pattern is the reference's. Called by whoever stores C: a launch of its own
+// after the GEMM took 2.5 us of every call (N = 5760, no such row).
+__device__ __forceinline__ float nonfinite_dot(const NonfiniteRows &nf, int row, int col) {
+    const float *xr = nf.x + (size_t)row * nf.ldx;
+    const int8_t *qr = nf.q + (size_t)col * nf.ldq;
+    float acc[8];
+#pragma unroll
+    for (int l = 0; l < 8; ++l) acc[l] = 0.0f;
+    int kk = 0;
+    for (; kk + 8 <= nf.K; kk += 8) {
+#pragma unroll
+        for (int l = 0; l < 8; ++l) acc[l] = __builtin_fmaf(xr[kk + l], (float)qr[kk + l], acc[l]);
+    }
+    float s = ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7]));
+    for (; kk < nf.K; ++kk) s += xr[kk] * (float)qr[kk];
+    return s;
+}
+
+// C = (in-order sum of ks k-slice partials [ks][M][N]) * scale (per column, or
+// none). With nf, rows whose factor is NaN are recomputed from it.
 int launch_gemv_reduce(const float *part, int ks, int M, int N, const float *scale, float *C,
-                       int ldc, hipStream_t st);
+                       int ldc, hipStream_t st, const NonfiniteRows &nf = NonfiniteRows{});
 
 // Full-K GEMV for decode batches of M <= 5 rows with fused row ops. Input:
 // bf16 term planes A [3][M][lda]; with ssp, the rows are RMSNorm inputs
@@ -296,6 +327,7 @@ struct GemmArgs {
     // 32t + 16 + j), formed in the epilogue from the scaled results (one
     // slice; N % 32 == 0)
     bool silu_pairs = false;
+    NonfiniteRows nf;  // int8 rows; unset: those rows come out NaN
 };
 int launch_gemm(const GemmArgs &a, hipStream_t st);
 // An [M][N] matrix left as ks ordered k-slices [ks][M][N] (row factors
@@ -308,11 +340,6 @@ struct Slices {
     size_t pst = 0;  // floats from one slice to the next (M * N)
     const float *scale = nullptr;
 };
-// Recomputes in f32 the rows of an int8-row GEMM whose factor a8s[i] is NaN
-// (non-finite inputs), giving the reference's +-inf / NaN pattern.
-int launch_gemm_i8_nonfinite_rows(const float *a, int lda, const int8_t *q, int ldq,
-                                  const float *scale, const float *a8s, float *c, int ldc, int M,
-                                  int N, int K, hipStream_t st);
 // Backend-table primitives and jit helpers (k_backend.hip). `part` holds
 // bk_reduce_work_floats() floats, `work` bk_max_work_bytes() bytes; the
 // scalar result goes to out[0] on the device.

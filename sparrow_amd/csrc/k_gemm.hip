@@ -24,6 +24,7 @@ struct GemmParams {
     float *part;        // k-slices > 1: raw sums times the row factor [ks][M][N]
     int group;          // tile order: 0 as dispatched, g > 0 XCD-grouped (gemm_tile)
     int silu;           // int8 rows: C = SiLU(gate) * up of interleaved pairs (GemmArgs)
+    NonfiniteRows nf;   // int8 rows: rows with a NaN factor (GemmArgs)
 };
 
 typedef __attribute__((__vector_size__(4 * sizeof(int)))) int gi32x4;
@@ -346,6 +347,14 @@ __global__ __launch_bounds__(64 * WMW * WNW) __attribute__((amdgpu_waves_per_eu(
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // copies past the end land before reuse
     __syncthreads();
 
+    // rows to recompute (the slice reduction does it where there are slices)
+    uint64_t nfm = 0;
+    static_assert(BM <= 64 && BN <= 128 && NW == 4, "a lane per row, two waves per column");
+    if (p.nf.f && ksl == 1) {
+        const float f = lane < BM && m0 + lane < p.M ? p.nf.f[m0 + lane] : 0.0f;
+        nfm = __ballot(!(f == f));
+    }
+
     // epilogue: the terms combined, 16-row slabs through LDS, 16-byte stores
     float *cs = (float *)smem + wave * 16 * C_LD;
     const bool vec = (p.ldc & 3) == 0 && ((uintptr_t)p.C & 15) == 0;
@@ -372,6 +381,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) __attribute__((amdgpu_waves_per_eu(
             const int row = m0 + wm * WM + i * 16 + rr_, col = n0 + wn * WN + c4;
             if (row >= p.M || col >= p.N) continue;
             const float rf = p.a8s[row];
+            if (nfm && !(rf == rf)) continue;  // below
             if (WN % 32 == 0 && p.silu) {
                 // the slab's 64 columns are two (16 gate, 16 up) pairs: a gate
                 // lane takes its up values 16 columns on, as silu_mul would
@@ -405,6 +415,12 @@ __global__ __launch_bounds__(64 * WMW * WNW) __attribute__((amdgpu_waves_per_eu(
         }
         __builtin_amdgcn_s_waitcnt(0xC07F);
         __builtin_amdgcn_wave_barrier();
+    }
+    // a thread per column, rows dealt to the two halves of the workgroup
+    for (int odd = wave >> 1; nfm; nfm &= nfm - 1, odd ^= 1) {
+        const int row = m0 + __builtin_ctzll(nfm), c = (wave & 1) * 64 + lane, col = n0 + c;
+        if (!odd && c < BN && col < p.N)
+            p.C[(size_t)row * p.ldc + col] = nonfinite_dot(p.nf, row, col) * p.scale[col];
     }
 }
 
@@ -477,69 +493,18 @@ static int launch_i8(const GemmParams &p, bool wb, int ksl, bool keep, hipStream
         gemm_dma_i8_kernel<BM, BN, NS, true, 2, WMW, WNW><<<grid, 64 * WMW * WNW, 0, st>>>(p);
     VMLM_HIP_CHECK(hipGetLastError());
     if (ksl == 1 || keep) return VMLM_OK;
-    return launch_gemv_reduce(p.part, ksl, p.M, p.N, p.scale, p.C, p.ldc, st);
+    return launch_gemv_reduce(p.part, ksl, p.M, p.N, p.scale, p.C, p.ldc, st, p.nf);
 }
 
 int gemm_i8_kslices(int M, int N, int K) {
     if (N % 4) return 1;  // the partial rows are written as 16-byte stores
     const int wgs = ((N + 127) / 128) * ((M + 63) / 64), nk = K / 64;
-    const int ks = wgs < 64 ? 4 : wgs < 160 ? 2 : 1;  // fill the 256 CUs
+    int ks = wgs < 64 ? 4 : wgs < 160 ? 2 : 1;  // fill the 256 CUs
+    // a long k over a small result: 200 x 2304 x 5760 (72 tiles) 38 -> 30 us (the
+    // slices stay within 8 MB, and the rows' terms at these sizes too, so what
+    // fitted the fixed scratch still does)
+    if (ks == 2 && wgs < 128 && nk >= 64 && M <= 256 && (size_t)M * N <= (size_t)1 << 19) ks = 4;
     return nk >= 8 * ks ? ks : 1;
-}
-
-// Rows of an int8-row GEMM whose factor is NaN (a NaN or infinite input,
-// q8_row_k) are recomputed here in f32 in the reference's order
-// (ops/src/kernels.rs:1256-1287: eight FMA lanes over k, the 8 -> 1 fold,
-// the scalar tail, then the scale), so their +-inf / NaN pattern is the
-// reference's. One thread per output column; each workgroup scans the row
-// factors 256 at a time into an LDS list and skips clean rows, so a GEMM
-// without such rows pays one short launch.
-__global__ __launch_bounds__(256) void gemm_i8_nonfinite_rows_kernel(
-    const float *__restrict__ a, int lda, const int8_t *__restrict__ q, int ldq,
-    const float *__restrict__ scale, const float *__restrict__ a8s, float *__restrict__ c,
-    int ldc, int M, int N, int K) {
-    __shared__ int list[256];
-    __shared__ int cnt;
-    const int j = blockIdx.x * 256 + threadIdx.x;
-    for (int base = 0; base < M; base += 256) {
-        if (threadIdx.x == 0) cnt = 0;
-        __syncthreads();
-        const int r = base + threadIdx.x;
-        if (r < M) {
-            const float f = a8s[r];
-            if (!(f == f)) list[atomicAdd(&cnt, 1)] = r;
-        }
-        __syncthreads();
-        const int n = cnt;
-        for (int e = 0; e < n && j < N; ++e) {
-            const int i = list[e];
-            const float *ar = a + (size_t)i * lda;
-            const int8_t *qr = q + (size_t)j * ldq;
-            float acc[8];
-#pragma unroll
-            for (int l = 0; l < 8; ++l) acc[l] = 0.0f;
-            int kk = 0;
-            for (; kk + 8 <= K; kk += 8) {
-#pragma unroll
-                for (int l = 0; l < 8; ++l)
-                    acc[l] = __builtin_fmaf(ar[kk + l], (float)qr[kk + l], acc[l]);
-            }
-            float s = ((acc[0] + acc[4]) + (acc[2] + acc[6])) + ((acc[1] + acc[5]) + (acc[3] + acc[7]));
-            for (; kk < K; ++kk) s += ar[kk] * (float)qr[kk];
-            c[(size_t)i * ldc + j] = s * scale[j];
-        }
-        __syncthreads();
-    }
-}
-
-int launch_gemm_i8_nonfinite_rows(const float *a, int lda, const int8_t *q, int ldq,
-                                  const float *scale, const float *a8s, float *c, int ldc, int M,
-                                  int N, int K, hipStream_t st) {
-    if (M <= 0 || N <= 0) return VMLM_OK;
-    gemm_i8_nonfinite_rows_kernel<<<(N + 255) / 256, 256, 0, st>>>(a, lda, q, ldq, scale, a8s, c,
-                                                                   ldc, M, N, K);
-    VMLM_HIP_CHECK(hipGetLastError());
-    return VMLM_OK;
 }
 
 int launch_gemm(const GemmArgs &a, hipStream_t st) {
@@ -581,6 +546,7 @@ int launch_gemm(const GemmArgs &a, hipStream_t st) {
                    (size_t)ksl * a.M * a.N, a.work_floats);
         p.part = a.work;
         p.silu = a.silu_pairs ? 1 : 0;
+        p.nf = a.nf;
         const int ns = a.stages ? a.stages : 2;
         // 64 x 128 tiles: 128-row tiles need 256 accumulator registers, run one
         // wave per SIMD and measured 30 % slower at the prefill shapes. Two

@@ -734,11 +734,13 @@ constexpr int RED_KS_MAX = 16;
 __global__ __launch_bounds__(256) void gemv_reduce_kernel(const float *__restrict__ part, int ks,
                                                           int M, int N,
                                                           const float *__restrict__ scale,
-                                                          float *__restrict__ C, int ldc) {
+                                                          float *__restrict__ C, int ldc,
+                                                          NonfiniteRows nf) {
     const int n = M * N;
     int i = blockIdx.x * 256 + threadIdx.x;
     const bool live = i < n;
     i = live ? i : n - 1;
+    const float rf = nf.f ? nf.f[i / N] : 0.0f;
     float v[RED_KS_MAX];
 #pragma unroll
     for (int s = 0; s < RED_KS_MAX; ++s) v[s] = part[(size_t)(s < ks ? s : ks - 1) * n + i];
@@ -748,15 +750,16 @@ __global__ __launch_bounds__(256) void gemv_reduce_kernel(const float *__restric
         if (s < ks) acc += v[s];
     if (!live) return;
     const int b = i / N, j = i % N;
+    if (!(rf == rf)) acc = nonfinite_dot(nf, b, j);
     C[(size_t)b * ldc + j] = scale ? acc * scale[j] : acc;
 }
 
 int launch_gemv_reduce(const float *part, int ks, int M, int N, const float *scale, float *C,
-                       int ldc, hipStream_t st) {
+                       int ldc, hipStream_t st, const NonfiniteRows &nf) {
     VMLM_GUARD(ks >= 1 && ks <= RED_KS_MAX && M >= 1 && N >= 1,
                "gemv reduce: 1 <= ks <= %d k-slices", RED_KS_MAX);
     const size_t n = (size_t)M * N;
-    gemv_reduce_kernel<<<cdiv(n, 256), 256, 0, st>>>(part, ks, M, N, scale, C, ldc);
+    gemv_reduce_kernel<<<cdiv(n, 256), 256, 0, st>>>(part, ks, M, N, scale, C, ldc, nf);
     VMLM_HIP_CHECK(hipGetLastError());
     return VMLM_OK;
 }

@@ -457,7 +457,8 @@ int launch_silu_q8(const float *part, int ks, int ldp, const float *sgu, int row
 // load. Lane piece p of a row: k-block p / 4, lane group g = p % 4, values
 // k = 64 (p / 4) + 8 g + 0..7 and 64 (p / 4) + 32 + 8 g + 0..7; rows past
 // the last (to the tile count) hold zero terms.
-// At least 2048 rows: rows_q8_wave_kernel (below), one launch. Between 256
+// At least 2048 rows: rows_q8_wave_kernel (below), one launch. Fewer, without a
+// norm or an add and up to RR_MAX elements: rows_q8_row_kernel. Else between 256
 // and 2048 rows: two launches. rows_q8_stats_kernel (one workgroup per row) finds
 // inv and the factor, rows_q8_terms_kernel (one workgroup per 16 rows x 32
 // lane pieces) forms y again with the same operations and writes the terms,
@@ -627,6 +628,68 @@ __global__ __launch_bounds__(16 * RQ_J) void rows_q8_terms_kernel(
 #pragma unroll
     for (int tt = 0; tt < Q8_T; ++tt)
         *(u32x4 *)(q8 + tt * plane + off) = u32x4{w[tt][0], w[tt][1], w[tt][2], w[tt][3]};
+}
+
+// Rows as they are (no norm, no residual add): one workgroup per row, a thread
+// a lane piece (16 values, whole 16-byte stores), one launch. The maximum is
+// exact in any order, so the terms are the other kernels' bits. 100 x 2304: 5.4
+// -> 4.3 us, 1000 x 2304: 11.6 (stats and terms) -> 9.8. Its 16-byte stores of
+// one row are 256 bytes apart: over many long rows the terms kernel's whole
+// blocks are faster (1000 x 5760: 17.1 against 13.7), hence RR_MAX.
+constexpr int RR_P = 2;  // lane pieces per thread: cols <= 8192
+constexpr size_t RR_MAX = 3600000;
+__global__ __launch_bounds__(256) void rows_q8_row_kernel(const float *__restrict__ x, int ldx,
+                                                          int cols, int rows, int row_tiles,
+                                                          float *__restrict__ q8s,
+                                                          int8_t *__restrict__ q8) {
+    __shared__ float sh[4];
+    const int row = blockIdx.x, tid = threadIdx.x, npc = cols >> 4, nkb = cols >> 6;
+    const size_t plane = (size_t)row_tiles * cols * 16;
+    auto piece_off = [&](int pc) {
+        return ((size_t)(row >> 4) * nkb + (pc >> 2)) * 1024 +
+               (size_t)((pc & 3) * 16 + (row & 15)) * 16;
+    };
+    const bool live = row < rows;
+    const float *xr = x + (size_t)(live ? row : 0) * ldx;
+    float4 v[RR_P][4];
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < RR_P; ++i) {
+        const int pc = tid + 256 * i;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            v[i][j] = live && pc < npc ? *(const float4 *)(xr + (pc >> 2) * 64 + 8 * (pc & 3) +
+                                                           32 * (j >> 1) + 4 * (j & 1))
+                                       : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < RR_P; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            mx = fmaxf(mx, fmaxf(fmaxf(q8_mag(v[i][j].x), q8_mag(v[i][j].y)),
+                                 fmaxf(q8_mag(v[i][j].z), q8_mag(v[i][j].w))));
+    const int k = q8_row_k(block_max256(mx, sh));
+    if (live && tid == 0) q8s[row] = q8_factor(k);
+#pragma unroll
+    for (int i = 0; i < RR_P; ++i) {
+        const int pc = tid + 256 * i;
+        if (pc >= npc) continue;
+        uint32_t w[Q8_T][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            int a[4][Q8_T];
+            q8_split(v[i][j].x, k, a[0]);
+            q8_split(v[i][j].y, k, a[1]);
+            q8_split(v[i][j].z, k, a[2]);
+            q8_split(v[i][j].w, k, a[3]);
+#pragma unroll
+            for (int tt = 0; tt < Q8_T; ++tt) w[tt][j] = pack_i8x4(a[0][tt], a[1][tt], a[2][tt], a[3][tt]);
+        }
+        const size_t off = piece_off(pc);
+#pragma unroll
+        for (int tt = 0; tt < Q8_T; ++tt)
+            *(u32x4 *)(q8 + tt * plane + off) = u32x4{w[tt][0], w[tt][1], w[tt][2], w[tt][3]};
+    }
 }
 
 // One launch for any row count: one wave per row, RW_ROWS rows per
@@ -830,6 +893,12 @@ int launch_rows_q8(const float *x, size_t ldx, const float *g, float eps, size_t
         else if (cols <= 1024 * 6) RW_LAUNCH(6);
         else RW_LAUNCH(8);
 #undef RW_LAUNCH
+        VMLM_HIP_CHECK(hipGetLastError());
+        return VMLM_OK;
+    }
+    if (!g && !ra && rows * cols <= RR_MAX) {
+        rows_q8_row_kernel<<<(unsigned)(tiles * 16), 256, 0, st>>>(
+            x, (int)ldx, (int)cols, (int)rows, (int)tiles, q8s, q8);
         VMLM_HIP_CHECK(hipGetLastError());
         return VMLM_OK;
     }

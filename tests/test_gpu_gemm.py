@@ -247,6 +247,34 @@ def test_gemm_direct_infinite_and_nan_rows(dev):
     assert np.abs(got[ok] - ref[ok]).max() <= 1e-5 * np.sqrt(np.mean(ref[ok] ** 2))
 
 
+# int8 rows: rows with a NaN or an infinity written by the GEMM's epilogue (odd N;
+# 96 columns a tile; the swizzled copy) and by the slice reduction; the rows' split
+# in one launch and in two (rows x K past 3.6e6), fewer and more k-slices.
+@pytest.mark.parametrize("m,n,k", [(129, 131, 256), (300, 2304, 128), (630, 64, 5760),
+                                   (150, 256, 2304), (200, 2048, 4096)])
+def test_gemm_int8_rows_infinite_and_nan_rows(dev, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    a, w, w64, s = direct_case(rng, m, n, k, True)
+    w[:20, 9] = 0
+    w64[:20, 9] = 0
+    rows = [0, 1, 62, 63, 64, 100, m - 2, m - 1]
+    a[rows[::2], 9] = np.inf
+    a[rows[1::2], k - 1] = -np.inf
+    a[64, 3] = np.nan
+    with np.errstate(invalid="ignore"):
+        ref = (a.astype(np.float64) @ w64.T) * s
+    c = dev.empty(m * n * 4)
+    dev.check(dev.lib.vmlm_hip_gemm_nt_int8(dev.up(a), dev.up(w), dev.up(s), c, m, n, k, None))
+    got = dev.down(c, (m, n), np.float32)
+    for f in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(f(got), f(ref))
+    ok = np.isfinite(ref)
+    # three int8 terms leave at most 2^-21 of the row's maximum per element
+    bound = (np.abs(np.where(np.isfinite(a), a, 0)).max(1)[:, None] * 2.0 ** -21 *
+             np.abs(w64).sum(1) * s + 1e-5 * np.sqrt(np.mean(ref[ok] ** 2)))
+    assert (np.abs(got.astype(np.float64) - ref)[ok] <= bound[ok]).all()
+
+
 # f32 GEMM: each tile (32 x 32, 32 x 64, 64 x 64, 128 x 128), rows and columns at
 # their edges, k at the 32-deep steps' edges, rows on and off 16 bytes (k % 4, n %
 # 4, operands a float off), with k-slices and without, NT and NN.
