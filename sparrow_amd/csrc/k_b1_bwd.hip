@@ -159,6 +159,89 @@ __global__ __launch_bounds__(256) void b1_bwd_t8_dw_v4_kernel(
     if (ok && h == 0) dw[e] = dw[e] + ((sm[0] + sm[1]) + (sm[2] + sm[3]));
 }
 
+// The same with the x rows through LDS: a wave takes up to 32 connections of
+// one output, copies 64 tokens of their rows straight into its own LDS (four
+// rows of 256 contiguous bytes an instruction, two chunks ahead) and reads
+// them back in the chains' order. The kernel above fetches 32 bytes of each of
+// 32 rows an instruction, two cycles a segment at the address unit, and a
+// wave's lines leave the L1 between its visits: 25 us at n = 1536, k0 = 32, t8
+// = 1024, here 13.8. Piece q of row r lies at q ^ 2 (r % 8): the sixteen lanes
+// that read a step of eight rows cover all banks once.
+constexpr int B1_DW_W = 2, B1_DW_NS = 3;           // waves of a workgroup, chunks in LDS
+constexpr int B1_DW_CHUNK = 32 * 256 + 256;        // 32 rows of x, one of dy
+__global__ __launch_bounds__(64 * B1_DW_W) void b1_bwd_t8_dw_lds_kernel(
+    const uint32_t *__restrict__ src, const float *__restrict__ xt, const float *__restrict__ dyt,
+    uint32_t t8, uint32_t n, uint32_t k0, float *__restrict__ dw, int *guard) {
+    __shared__ __align__(16) uint8_t lds[B1_DW_W * B1_DW_NS * B1_DW_CHUNK];
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t grp = (k0 + 31) / 32, gw = blockIdx.x * B1_DW_W + wave, j = gw / grp;
+    if (j >= n) return;  // whole waves; no barriers below
+    const int c = lane >> 1, h = lane & 1;
+    const uint32_t idx = gw % grp * 32 + c;
+    const bool live = idx < k0;
+    const size_t e = (size_t)j * k0 + (live ? idx : 0);
+    const uint32_t s = src[e];
+    const bool ok = live && s < n;
+    if (live && !ok && h == 0) atomicOr(guard, 1);
+    const uint32_t row = (ok ? s : 0u) * t8 * 4;  // bytes; n * t8 * 4 < 2^32
+    // copy v: rows 4v + lane / 16, the lane bringing piece lane % 16 as placed
+    uint32_t voff[8];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) voff[v] = (uint32_t)__shfl((int)row, 8 * v + 2 * (lane >> 4), 64);
+    const uint32_t pc[2] = {(uint32_t)((lane & 15) ^ (2 * (lane >> 4))),
+                            (uint32_t)((lane & 15) ^ (2 * (lane >> 4) + 8))};
+    const float *dr = dyt + (size_t)j * t8;
+    const uint8_t *mine = lds + wave * (B1_DW_NS * B1_DW_CHUNK);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(mine));
+    const uint32_t nch = (t8 + 63) / 64;
+    auto issue = [&](uint32_t kt) {  // nine copies; tokens past the row's end repeat its last
+        const uint32_t base = lds0 + kt % B1_DW_NS * B1_DW_CHUNK;
+        uint32_t tb[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) tb[i] = 4 * min(kt * 64 + 4 * pc[i], t8 - 4);
+#pragma unroll
+        for (int v = 0; v < 8; ++v) dma16s(xt, voff[v] + tb[v & 1], base + v * 1024);
+        if (lane < 16) dma16s(dr, 4 * min(kt * 64 + 4 * (uint32_t)lane, t8 - 4), base + 8192);
+    };
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    issue(0);
+    if (nch > 1) issue(1);
+    for (uint32_t kt = 0; kt < nch; ++kt) {
+        if (kt + 2 < nch) {
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // the reads of the chunk written next
+            issue(kt + 2);
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(18));
+        } else if (kt + 1 < nch) {
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(9));
+        } else {
+            __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+        }
+        asm volatile("" ::: "memory");
+        const uint8_t *st = mine + kt % B1_DW_NS * B1_DW_CHUNK;
+        auto step = [&](int u) {
+            const float4 a = *(const float4 *)(st + 8192 + u * 32 + h * 16);
+            const float4 b = *(const float4 *)(st + c * 256 + (u ^ (c & 7)) * 32 + h * 16);
+            acc[0] = __builtin_fmaf(a.x, b.x, acc[0]);
+            acc[1] = __builtin_fmaf(a.y, b.y, acc[1]);
+            acc[2] = __builtin_fmaf(a.z, b.z, acc[2]);
+            acc[3] = __builtin_fmaf(a.w, b.w, acc[3]);
+        };
+        const int steps = (int)min(t8 - kt * 64, 64u) / 8;
+        if (steps == 8) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) step(u);
+        } else {
+            for (int u = 0; u < steps; ++u) step(u);
+        }
+    }
+    // hsum256: l and l + 4 sit in neighbouring lanes
+    float sm[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sm[q] = acc[q] + dpp_mov<0xB1>(acc[q]);
+    if (ok && h == 0) dw[e] = dw[e] + ((sm[0] + sm[1]) + (sm[2] + sm[3]));
+}
+
 // t8 dx: one thread per (source, token): dxt[s][p] = fma(dyt[i][p], w[e],
 // dxt[s][p]) over the source's connections in ascending e.
 __global__ __launch_bounds__(256) void b1_bwd_t8_dx_kernel(const uint2 *__restrict__ pairs,
@@ -517,7 +600,13 @@ int launch_b1_backward_t8(const float *w, const uint32_t *src, const float *xt, 
     RevIndex r;
     int rc = build_rev(src, w, E, k0, d, work, r, st);
     if (rc) return rc;
-    if ((((uintptr_t)xt | (uintptr_t)dyt) & 15) == 0)
+    const bool al = (((uintptr_t)xt | (uintptr_t)dyt) & 15) == 0;
+    // whole groups of 32 connections, or nearly (a wave takes a group)
+    const size_t grp = (k0 + 31) / 32;
+    if (al && n * t8 <= 0x3fffffff && n * grp <= 0x3fffffff && k0 * 4 >= grp * 96)
+        b1_bwd_t8_dw_lds_kernel<<<cdiv(n * grp, B1_DW_W), 64 * B1_DW_W, 0, st>>>(
+            src, xt, dyt, (uint32_t)t8, (uint32_t)n, (uint32_t)k0, dw, guard_flag_ptr());
+    else if (al)
         b1_bwd_t8_dw_v4_kernel<<<bwd_blocks(E * 2), 256, 0, st>>>(src, xt, dyt, t8, E, (uint32_t)k0,
                                                                   d, dw, guard_flag_ptr());
     else

@@ -246,3 +246,31 @@ def test_b1_backward_guards(hip):
         ops.b1_backward_t8(w, np.zeros((4, 2), np.uint32), np.ones((4, 12), np.float32),
                            np.ones((4, 12), np.float32))
     assert e.value.code == 9  # t8 not a multiple of 8
+
+
+# dw through LDS (k0 at least three quarters of its groups of 32): t8 at and off
+# the 64-token chunks, one to four chunks and a remainder, groups that are not
+# full, more groups than one per output; an id past n is skipped.
+@pytest.mark.parametrize("n,k0,t8", [(70, 24, 8), (33, 31, 72), (101, 32, 64), (71, 49, 200),
+                                     (65, 64, 136), (1, 32, 256)])
+def test_b1_backward_t8_dw_lds_bitwise(hip, oracle, n, k0, t8):
+    from sparrow_amd.conn import DeviceBuffer
+    rng = np.random.default_rng(n + k0 + t8)
+    w = rng.standard_normal((n, k0)).astype(np.float32)
+    src = rng.integers(0, n, size=(n, k0)).astype(np.uint32)
+    xt, dyt, dxt0 = (rng.standard_normal((n, t8)).astype(np.float32) for _ in range(3))
+    dw0 = rng.standard_normal((n, k0)).astype(np.float32)
+    bad = src.copy()
+    bad[n - 1, k0 - 1] = n
+    ref_w = w.copy()
+    ref_w[n - 1, k0 - 1] = 0.0  # the connection adds nothing to dx (+-0)
+    dev = [DeviceBuffer.from_array(a) for a in (w, bad, xt, dyt, dxt0, dw0)]
+    assert hip.vmlm_hip_b1_backward_t8(*[d.ptr for d in dev[:4]], t8, n, k0, dev[4].ptr,
+                                       dev[5].ptr, None) == 0
+    assert hip.vmlm_hip_check_guards() == 9
+    ox, ow = oracle.b1_backward_t8(ref_w, src, xt, dyt, dxt0, dw0)
+    ow[n - 1, k0 - 1] = dw0[n - 1, k0 - 1]
+    assert np.array_equal(bits(dev[5].to_array((n, k0), np.float32)), bits(ow))
+    assert np.array_equal(dev[4].to_array((n, t8), np.float32), ox)
+    for d in dev:
+        d.free()
