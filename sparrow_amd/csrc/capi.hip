@@ -320,8 +320,14 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
             return fail(VMLM_ERR_UNIMPL, "q8/bf16 GEMM with K %% 128 != 0 or unaligned weights "
                                          "stages a padded weight copy and cannot be captured");
     }
+    // (a result over its own operands takes a path that has read them before
+    // the first store: term planes, int8 rows or a padded copy)
+    auto over = [&](const void *x, size_t bytes) {
+        return (uintptr_t)c < (uintptr_t)x + bytes && (uintptr_t)x < (uintptr_t)c + m * n * 4;
+    };
+    const bool alias = over(a, m * k * 4) || over(W, n * k * esz);
     const bool few = wi8 && m <= 16 && !padded && ((uintptr_t)a & 15) == 0;
-    if (!few && q_direct(wi8, padded, m, n, k)) {
+    if (!few && !alias && q_direct(wi8, padded, m, n, k)) {
         // the fixed scratch keeps its limit of shapes, whichever path they take
         if constexpr (!std::is_same<WS, Stage>::value) {
             if (padded) stg.template alloc<uint8_t>(n * Kp * esz);

@@ -302,3 +302,24 @@ def test_gemm_f32_edges(dev, m, n, k):
                 dev.check(f(da, db, dc, m, n, k, acc, None))
                 got = dev.down(dc, (m, n), np.float32).astype(np.float64)
                 assert (np.abs(got - (ref + c0 if acc else ref)) <= bound).all()
+
+
+@pytest.mark.parametrize("m,k,int8", [(77, 1001, True), (17, 256, True), (9, 384, False)])
+def test_gemm_over_its_own_rows(dev, m, k, int8):
+    """The result written over the activation rows (n = k): every row is read
+    before the first store, so it is the result in a buffer of its own."""
+    rng = np.random.default_rng(m * 3 + k)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    s = np.full(k, 0.01, np.float32)
+    if int8:
+        w = rng.integers(-127, 128, (k, k), dtype=np.int8)
+        ref = (a.astype(np.float64) @ w.astype(np.float64).T) * s
+    else:
+        w = bf16_bits(rng.standard_normal((k, k), dtype=np.float32))
+        ref = a.astype(np.float64) @ bf16_value(w).astype(np.float64).T
+    c = dev.up(a)
+    if int8:
+        dev.check(dev.lib.vmlm_hip_gemm_nt_int8(c, dev.up(w), dev.up(s), c, m, k, k, None))
+    else:
+        dev.check(dev.lib.vmlm_hip_gemm_nt_bf16(c, dev.up(w), c, m, k, k, None))
+    assert_close_rms(dev.down(c, (m, k), np.float32), ref)
