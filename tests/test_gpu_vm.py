@@ -870,3 +870,43 @@ def test_vm_row_kernels_past_one_grid(gvm):
         g.write("x", xv)
         g.run()
         assert np.array_equal(bits(g.read("y").ravel()), bits(wv * xv))
+
+
+def test_vm_prints_in_order(gvm, oracle):
+    """PRINTs that wait in the host block (inside a counted loop, before a
+    jump), one that does not fit what is left of it, one larger than all of
+    it, and the first ones of a run that a guard ends: the values in program
+    order, as the oracle's."""
+    rng = np.random.default_rng(5)
+    P = vmb.Program()
+    n, one = P.scalar("n", 3.0), P.scalar("one", 1.0)
+    acc = P.act("acc", 1, 1)
+    rows = [P.const(f"x{i}", rng.standard_normal((1, c)).astype(np.float32))
+            for i, c in enumerate((257, 1, 300_000, 300_001, 600_000, 64))]
+    top = P.label()
+    P.ins("EWADD", acc, acc, one)
+    P.ins("PRINT", acc)
+    P.ins("PRINT", rows[0])
+    P.ins("LOOP_CNT", top, n)
+    P.ins("PRINT", acc)
+    P.ins("EWADD", acc, acc, one)  # after the print: it keeps the old value
+    for r in rows[1:]:
+        P.ins("PRINT", r)
+    P.ins("PRINT", acc)
+    P.ins("HALT")
+    (g, _), (o, _) = both(gvm, P)
+    assert np.array_equal(bits(g), bits(o))
+
+    from sparrow_amd import VmlmError
+    P = vmb.Program()
+    x = P.const("x", np.float32([[1, 2, 3, 4]]))
+    small = P.act("small", 1, 2)
+    P.ins("PRINT", x)
+    P.ins("COPY", small, x)
+    P.ins("HALT")
+    with gvm.Vm(P.build()) as v:
+        for _ in range(2):
+            v.clear_output()
+            with pytest.raises(VmlmError):
+                v.run()
+            assert np.array_equal(v.output(), np.float32([1, 2, 3, 4]))
