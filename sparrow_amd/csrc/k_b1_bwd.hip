@@ -277,6 +277,20 @@ __global__ __launch_bounds__(B1_DX_THREADS) void b1_bwd_t8_dx_lds_kernel(
     constexpr int Q = TB / 4, SRC = B1_DX_THREADS / Q;  // lanes per source, sources per pass
     const int tid = threadIdx.x, q = tid % Q;
     const size_t t0 = (size_t)blockIdx.x * TB;
+    const size_t t = t0 + 4 * (size_t)q;
+    const int s1 = min(d, ((int)blockIdx.y + 1) * per);
+    // the first source's range, then its first pairs, while the tile arrives
+    int s = (int)blockIdx.y * per + tid / Q;
+    uint32_t c = 0, end = 0;
+    if (s < s1) {
+        c = off[s];
+        end = off[s + 1];
+    }
+    // pairs c .. c + 3 of a source that ends at e (past it the last, not used)
+    auto load_pairs = [&](uint32_t c, uint32_t e, uint2 (&p)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = pairs[c + u < e ? c + u : e ? e - 1 : 0];
+    };
     // stage row r's tokens t0 .. t0 + TB - 1 (t8 is a multiple of 8: a quad is
     // all in range or all out), eight pieces in flight
     const int npc = d * Q;
@@ -294,19 +308,25 @@ __global__ __launch_bounds__(B1_DX_THREADS) void b1_bwd_t8_dx_lds_kernel(
             if (pc < npc) b1_dx_tile[pc] = v[k];
         }
     }
+    uint2 p[4];
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    load_pairs(c, end, p);
+    if (s < s1 && t < t8) acc = *(const float4 *)(dxt + (size_t)s * t8 + t);
     __syncthreads();
-    const size_t t = t0 + 4 * (size_t)q;
     if (t >= t8) return;
-    const int s1 = min(d, ((int)blockIdx.y + 1) * per);
-    for (int s = (int)blockIdx.y * per + tid / Q; s < s1; s += SRC) {
-        float4 *o = (float4 *)(dxt + (size_t)s * t8 + t);
-        float4 acc = *o;
-        const uint32_t end = off[s + 1];
-        for (uint32_t c = off[s]; c < end; c += 4) {
-            uint2 p[4];
+    while (s < s1) {
+        const int sn = s + SRC;
+        uint32_t nc = 0, nend = 0;
+        float4 nacc = acc;
+        if (sn < s1) {
+            nc = off[sn];
+            nend = off[sn + 1];
+            nacc = *(const float4 *)(dxt + (size_t)sn * t8 + t);
+        }
+        for (; c < end; c += 4) {
+            uint2 np[4];
             float4 v[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) p[u] = pairs[c + u < end ? c + u : end - 1];
+            load_pairs(c + 4, end, np);
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = b1_dx_tile[p[u].x * Q + q];
 #pragma unroll
@@ -318,8 +338,15 @@ __global__ __launch_bounds__(B1_DX_THREADS) void b1_bwd_t8_dx_lds_kernel(
                     acc.z = __builtin_fmaf(v[u].z, w, acc.z);
                     acc.w = __builtin_fmaf(v[u].w, w, acc.w);
                 }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) p[u] = np[u];
         }
-        *o = acc;
+        *(float4 *)(dxt + (size_t)s * t8 + t) = acc;
+        s = sn;
+        c = nc;
+        end = nend;
+        acc = nacc;
+        load_pairs(c, end, p);
     }
 }
 
