@@ -910,3 +910,19 @@ def test_vm_prints_in_order(gvm, oracle):
             with pytest.raises(VmlmError):
                 v.run()
             assert np.array_equal(v.output(), np.float32([1, 2, 3, 4]))
+
+
+@pytest.mark.parametrize("r,ac,bc", [(1, 1, 1), (3, 5, 64), (65, 300, 7), (2, 70_001, 3)])
+def test_vm_concat_in_one_launch(gvm, oracle, r, ac, bc):
+    """CONCAT of halves of unlike widths: one launch whose grid is sized by the
+    larger half."""
+    rng = np.random.default_rng(r + ac)
+    P = vmb.Program()
+    a = P.const("a", rng.standard_normal((r, ac)).astype(np.float32))
+    b = P.const("b", rng.standard_normal((r, bc)).astype(np.float32))
+    y = P.act("y", r, ac + bc)
+    P.ins("CONCAT", y, a, b)
+    P.ins("PRINT", y)
+    P.ins("HALT")
+    (g, _), (o, _) = both(gvm, P)
+    assert np.array_equal(bits(g), bits(o))
