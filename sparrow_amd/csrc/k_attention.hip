@@ -1198,15 +1198,23 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(DecodeArgs a, floa
             if (grp == 0) *(float4 *)&pc[4 + 4 * q] = o;
         }
     };
-    while (s < s1) {
+    // Two sub-chunks, the next one's rows requested before each; false: done.
+    // A loop's header waits for every load in flight, so the next rows would be
+    // requested only when the current ones have arrived: the first four of a
+    // wave are straight code.
+    auto two = [&]() -> bool {
         load(kb, vb, live(s + NW));
         consume(ka, va, s);
         s += NW;
-        if (s >= s1) break;
+        if (s >= s1) return false;
         load(ka, va, live(s + NW));
         consume(kb, vb, s);
         s += NW;
-    }
+        return s < s1;
+    };
+    if (s < s1 && two() && two())
+        while (two()) {
+        }
     if constexpr (SPLIT) return;  // merged by attn_decode_merge_kernel
     __syncthreads();
     const int nloc = s1 - s0;  // this workgroup's sub-chunks (all of them unless nf)
