@@ -156,10 +156,11 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectParams p) {
     }
 
     // one row of tiles: the second and third terms' products in an accumulator
-    // of their own (NA = 2), a third of the roundings at the sum's magnitude,
-    // as the few-row GEMV has them (2 x 2048 x 2122: relative
-    // error 1.7e-7 -> 8e-8)
-    constexpr int NA = TM == 1 ? 2 : 1;
+    // of their own, and the first term's two halves of a block in one each: half
+    // the roundings at the sum's magnitude, no more than the few-row GEMV's
+    // shorter runs of k have (with the halves in one, 2 x 19728 x 1536 bf16 had a
+    // relative error of 1.18e-7 against its 9.9e-8)
+    constexpr int NA = TM == 1 ? 3 : 1;
     f32x4 acc[NA][TM][TN];
 #pragma unroll
     for (int n = 0; n < NA; ++n)
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectParams p) {
                 for (int s = 0; s < 3; ++s)
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
-                        f32x4 &c = acc[s == 0 ? 0 : NA - 1][i][j];
+                        f32x4 &c = acc[s == 0 && NA > 1 ? h : NA - 1][i][j];
                         c = dg_mfma(t[h][s], wf[j][h], c);
                     }
         }
@@ -276,7 +277,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_direct_kernel(DirectParams p) {
 #pragma unroll
         for (int j = 0; j < TN; ++j)
             red[(wave * TM * TN + i * TN + j) * 64 + lane] =
-                NA == 2 ? acc[0][i][j] + acc[NA - 1][i][j] : acc[0][i][j];
+                NA > 1 ? (acc[0][i][j] + acc[NA / 2][i][j]) + acc[NA - 1][i][j] : acc[0][i][j];
     __syncthreads();
     // accumulator (4g + e, r) of a tile: four rows of one column per thread
     for (int u = tid; u < TM * TN * 64; u += NW * 64) {
