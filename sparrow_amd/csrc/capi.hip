@@ -275,20 +275,25 @@ static inline size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; 
 //    three launches, 7 + 0.2 per k-step and the products at 500 TFLOP/s (17 x 2304 x 2304: 17.0 -> 7.2; 64 x 5760 x 2304: 21.1 ->
 //    15.8; 100 x 2304 x 5760: 27.6 -> 20.5); up to 128 rows, above which the
 //    row blocks of the int8 GEMM are full (300 x 5760 x 2304: 39 against 44);
-//  * else the padded weight copy, the term planes and the bf16 GEMM: 10, the
-//    copy at 4 TB/s, and 1.2 per k-step of one tile or the products at 230
-//    TFLOP/s (77 x 1537 x 1001 int8: 30.1 -> 6.6; 1000 x 1500 x 1100: 33.5 ->
-//    22.9; 333 x 1537 x 1536 bf16: 27.5 -> 15.3; 60 x 40509 x 2304 bf16 stays,
-//    66 to 78).
+//  * else the term planes and the bf16 GEMM: 10, and 0.7 per k-step of one tile
+//    or the products at 230 TFLOP/s; with the padded weight copy the copy at 4
+//    TB/s and, from K = 512, 8 more for its launches (below, the store of C is
+//    much of the direct kernel's time and its estimate too low: 768 x 11520 x 369
+//    int8 stays, 55 to 62) (77 x 1537 x 1001 int8: 30.1 -> 6.6; 1000 x
+//    1500 x 1100: 33.5 -> 22.9; 333 x 1537 x 1536 bf16: 27.5 -> 15.3; 44 x 23698 x
+//    2304 bf16 stays, 34 to 50, and 60 x 40509 x 2304, 66 to 78). The estimate of
+//    the direct kernel is low by a tenth at most sizes near the line (1181 x 1536
+//    x 2328 int8 stays: 56 to 60).
 static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
     if (k == 0 || m > 4096 || n > (size_t)1 << 24 || k > (size_t)1 << 24) return false;
     const double us = gemm_direct_us((int)m, (int)n, (int)k, wi8);
     const double nk = (double)((k + 63) / 64), flop = 2.0 * m * n * k;
     if (!padded && wi8) return m > 16 && m <= 128 && us < 7.0 + 0.2 * nk + flop / 500e6;
     if (!padded && m <= 16) return m > 5 || us < 20.0;
-    const double steps = 1.2 * nk, prod = flop / 230e6;
-    const double copy = padded ? 2.0 * n * k * (wi8 ? 1 : 2) / 4e6 : 0.0;
-    return us < 10.0 + copy + (steps > prod ? steps : prod);
+    const double steps = 0.7 * nk, prod = flop / 230e6;
+    const double copy =
+        padded ? (k >= 512 ? 8.0 : 0.0) + 2.0 * n * k * (wi8 ? 1 : 2) / 4e6 : 0.0;
+    return 1.1 * us < 10.0 + copy + (steps > prod ? steps : prod);
 }
 
 // int8 / bf16 weight GEMM on device operands: C[m,n] = A[m,k] . W[n,k]^T (* scale).
