@@ -389,11 +389,13 @@ constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 
 // Issued as inline assembly so that the compiler does not order every later
 // LDS read behind it; the callers wait for the copies with explicit vmcnt
 // waits and publish them with barriers. m0 is not used by anything else in
-// the kernels that use these.
+// the kernels that use these. A write of m0 needs one wait state before a load
+// into LDS reads it; the compiler fills none inside an assembly string, so the
+// s_nop is part of it.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved; nothing else here uses it
 __device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :
                  : "v"(gptr), "s"(lds_base)
                  : "memory", "m0");
@@ -403,7 +405,7 @@ __device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base) {
 // per-lane byte offset: one VGPR per distinct offset instead of a 64-bit
 // address per copy.
 __device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(voff), "s"(sbase), "s"(lds_base)
                  : "memory", "m0");
