@@ -213,7 +213,11 @@ int vmlm_attention_decode_split(const float *q, const float *k_new, const float 
                                 float scale, int split);
 
 /* ================================================================ layer 2
- * Device pointers, asynchronous on `stream`. Same semantics as layer 1. */
+ * Device pointers, asynchronous on `stream`. Same semantics as layer 1.
+ * The result of the int8 and bf16 weight GEMMs may lie over their operands (C
+ * is then formed in the workspace; where the fixed scratch of the noalloc call
+ * has no room for it, a row of A under C with a NaN or an infinity comes out
+ * NaN, and weights under C are refused with 9 unless they are staged). */
 int vmlm_hip_gemm_nt_int8(const float *a, const int8_t *q, const float *scale, float *c,
                           size_t m, size_t n, size_t k, void *stream);
 /* The same GEMM with no device allocation: no counterpart in the

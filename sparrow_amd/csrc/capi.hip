@@ -306,11 +306,15 @@ static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
 // scratch array of the allocation-free entry point (ScratchBump). Wsw, when
 // given, is a swizzled copy of int8 W (launch_swizzle_w) that the caller
 // keeps: the small-row launch and the int8-row GEMM read it instead of W.
+// `over`: C lies over A or W all the same (q_matmul, below); only what has read
+// that operand before its first store is taken then.
+struct QOver {
+    bool a = false, w = false;
+};
 template <class WS>
-static int q_matmul(const float *a, const void *W, bool wi8, const float *scale, float *c,
-                    size_t m, size_t n, size_t k, hipStream_t st, WS &stg,
-                    const void *Wsw = nullptr) {
-    if (m == 0 || n == 0) return VMLM_OK;
+static int q_matmul_to(const float *a, const void *W, bool wi8, const float *scale, float *c,
+                       size_t m, size_t n, size_t k, hipStream_t st, WS &stg, const void *Wsw,
+                       QOver over = QOver{}) {
     const size_t esz = wi8 ? 1 : 2;
     const size_t Kp = round_up(k == 0 ? 1 : k, 128);  // one 128-byte GEMV chunk covers 128 k
     const bool padded = Kp != k || ((uintptr_t)W & 15);
@@ -325,12 +329,7 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
             return fail(VMLM_ERR_UNIMPL, "q8/bf16 GEMM with K %% 128 != 0 or unaligned weights "
                                          "stages a padded weight copy and cannot be captured");
     }
-    // (a result over its own operands takes a path that has read them before
-    // the first store: term planes, int8 rows or a padded copy)
-    auto over = [&](const void *x, size_t bytes) {
-        return (uintptr_t)c < (uintptr_t)x + bytes && (uintptr_t)x < (uintptr_t)c + m * n * 4;
-    };
-    const bool alias = over(a, m * k * 4) || over(W, n * k * esz);
+    const bool alias = over.a || over.w;
     const bool few = wi8 && m <= 16 && !padded && ((uintptr_t)a & 15) == 0;
     if (!few && !alias && q_direct(wi8, padded, m, n, k)) {
         // the fixed scratch keeps its limit of shapes, whichever path they take
@@ -373,7 +372,7 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
     // int8 weights, up to FX_ROWS rows: one full-K launch whose waves split
     // their k-runs of the f32 rows into int8 terms themselves
     if (wi8 && m <= FX_ROWS && Wd == W && ((uintptr_t)a & 15) == 0 && k <= (size_t)1 << 30 &&
-        fx_run_blocks((int)k)) {
+        !alias && fx_run_blocks((int)k)) {
         FxArgs x;
         x.W = Wsw ? Wsw : Wd;
         x.swizzled = Wsw != nullptr;
@@ -393,7 +392,7 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
     const size_t nch = Kp / 128;
     const int nc = nch % 2 == 0 ? 2 : nch % 3 == 0 ? 3 : 1;
     if (wi8 && m <= 16 && Wd == W && k % 4 == 0 && ((uintptr_t)a & 15) == 0 &&
-        nch / nc <= 16) {
+        nch / nc <= 16 && !(alias && nch == (size_t)nc)) {
         const int ks = (int)(nch / nc);
         float *part = ks > 1 ? stg.template alloc<float>((size_t)ks * m * n) : nullptr;
         STAGE_OK(stg);
@@ -424,7 +423,7 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
     }
     // int8 weights, many rows, unpadded K: the rows as int8 terms with a
     // per-row factor, then the int8 x int8 MFMA GEMM
-    if (wi8 && m > 16 && Wd == W && Kp == k && k <= 8192 && ((uintptr_t)a & 15) == 0) {
+    if (wi8 && m > 16 && Wd == W && Kp == k && k <= 8192 && ((uintptr_t)a & 15) == 0 && !over.w) {
         int8_t *a8 = stg.template alloc<int8_t>(q8_rows_bytes(m, k));
         float *a8s = stg.template alloc<float>(m);
         const size_t gw = gemm_i8_work_floats((int)m, (int)n, (int)k);
@@ -446,7 +445,7 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
         GemmArgs g;
         g.W = Wsw ? Wsw : blk ? (const void *)wsw : Wd;
         g.w_blocked = blk;
-        g.nf.f = a8s;
+        g.nf.f = over.a ? nullptr : a8s;  // (rows under C: gone when they are recomputed)
         g.nf.x = a;
         g.nf.q = (const int8_t *)Wd;
         g.nf.ldx = g.nf.ldq = g.nf.K = (int)k;
@@ -464,6 +463,8 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
         g.ldc = (int)n;
         return launch_gemm(g, st);
     }
+    if (over.w && Wd == W)
+        return fail(VMLM_ERR_GUARD, "q8/bf16 GEMM over its own weights: C does not fit the workspace");
     uint16_t *terms = stg.template alloc<uint16_t>((size_t)T * m * Kp);
     STAGE_OK(stg);
     int rc = launch_split_terms(a, k, (int)m, (int)k, T, terms, (int)Kp, st);
@@ -496,6 +497,40 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
     g.Y = c;
     g.ldy = (int)n;
     return launch_gemv(g, st);
+}
+
+// The GEMM with C anywhere. Over its own operands C is formed in the workspace
+// and copied: the launches store while other workgroups still read the weights,
+// the scales and the f32 rows (of a few-row call, and the rows with a NaN or an
+// infinity of any). A fixed scratch that holds the path's own workspace and not
+// C as well keeps what it took before: the paths that have read their rows (and
+// a padded copy of W) by the first store, where a row under C with a NaN or an
+// infinity comes out NaN.
+template <class WS>
+static int q_matmul(const float *a, const void *W, bool wi8, const float *scale, float *c,
+                    size_t m, size_t n, size_t k, hipStream_t st, WS &stg,
+                    const void *Wsw = nullptr) {
+    if (m == 0 || n == 0) return VMLM_OK;
+    auto over = [&](const void *x, size_t bytes) {
+        return (uintptr_t)c < (uintptr_t)x + bytes && (uintptr_t)x < (uintptr_t)c + m * n * 4;
+    };
+    const QOver o{over(a, m * k * 4), over(W, n * k * (wi8 ? 1 : 2))};
+    const bool os = scale && over(scale, n * 4);
+    if (!o.a && !o.w && !os) return q_matmul_to(a, W, wi8, scale, c, m, n, k, st, stg, Wsw);
+    auto beside = [&]() {
+        float *t = stg.template alloc<float>(m * n);
+        STAGE_OK(stg);
+        const int rc = q_matmul_to(a, W, wi8, scale, t, m, n, k, st, stg, Wsw);
+        return rc ? rc : launch_copy(c, t, m * n, st);
+    };
+    if constexpr (std::is_same<WS, Stage>::value) return beside();
+    else {
+        const WS was = stg;
+        const int rc = beside();
+        if (!stg.status || os) return rc;
+        stg = was;
+        return q_matmul_to(a, W, wi8, scale, c, m, n, k, st, stg, Wsw, o);
+    }
 }
 
 // The int8 GEMM of the device VM, which keeps swizzled copies of its int8

@@ -368,6 +368,7 @@ int launch_b1_backward_t8(const float *w, const uint32_t *src, const float *xt, 
                           hipStream_t st);
 // Zero-fills `bytes` bytes with a kernel (capturable, unlike hipMemsetAsync).
 int launch_fill_zero(void *p, size_t bytes, hipStream_t st);
+int launch_copy(float *dst, const float *src, size_t n, hipStream_t st);
 int gemm_i8_kslices(int M, int N, int K);
 inline size_t gemm_i8_work_floats(int M, int N, int K) {
     const int ks = gemm_i8_kslices(M, N, K);

@@ -1101,6 +1101,21 @@ int launch_scale(float *dst, const float *src, size_t n, float s, hipStream_t st
     return VMLM_OK;
 }
 
+// A copy as a kernel, for the same reason as the zero fill below.
+__global__ __launch_bounds__(256) void copy_kernel(float *__restrict__ d,
+                                                   const float *__restrict__ s, size_t n) {
+    const size_t stride = (size_t)gridDim.x * 256;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) d[i] = s[i];
+}
+
+int launch_copy(float *dst, const float *src, size_t n, hipStream_t st) {
+    if (n == 0) return VMLM_OK;
+    const unsigned blocks = cdiv(n, 256);
+    copy_kernel<<<blocks > 4096 ? 4096 : blocks, 256, 0, st>>>(dst, src, n);
+    VMLM_HIP_CHECK(hipGetLastError());
+    return VMLM_OK;
+}
+
 // Zero fill as a kernel, so that a caller's stream capture records only
 // kernel nodes. `head` bytes up to the first 16-byte boundary, `n16` 16-byte
 // stores, then `tail` bytes.

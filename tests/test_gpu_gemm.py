@@ -323,3 +323,55 @@ def test_gemm_over_its_own_rows(dev, m, k, int8):
     else:
         dev.check(dev.lib.vmlm_hip_gemm_nt_bf16(c, dev.up(w), c, m, k, k, None))
     assert_close_rms(dev.down(c, (m, k), np.float32), ref)
+
+
+# every path of the int8 / bf16 GEMM: full-K and k-split GEMV, one slice and more;
+# one launch; int8 rows without and with k-slices, weights in rows and swizzled;
+# term planes over weights as they are and over a padded copy
+@pytest.mark.parametrize("m,k,int8,over", [
+    (m, k, int8, over)
+    for m, k, int8 in [(3, 2304, True), (16, 384, True), (9, 2304, True), (77, 1001, True),
+                       (300, 512, True), (150, 256, True), (1600, 2304, True), (4100, 130, True),
+                       (300, 640, False), (3, 1024, False), (1000, 770, False)]
+    for over in ("rows", "weights", "scales")[:3 if int8 else 2]])
+def test_gemm_over_any_operand(dev, m, k, int8, over):
+    """The result written over an operand (n = k) has the bits of the result in a
+    buffer of its own, rows with an infinity or a NaN included."""
+    rng = np.random.default_rng(m * 5 + k)
+    a, w, _, s = direct_case(rng, m, k, k, int8)
+    a[m - 1, 5] = np.inf
+    a[m // 2, k - 1] = np.nan
+    size = max(m * k * 4, k * k * 2)
+
+    def put(x):
+        p = dev.empty(size)
+        dev.check(dev.lib.vmlm_hip_memcpy_h2d(p, np.ascontiguousarray(x).ctypes.data, x.nbytes))
+        return p
+
+    out = []
+    for own in (True, False):
+        da, dw, ds = put(a), put(w), put(s) if int8 else None
+        c = dev.empty(size) if own else dict(rows=da, weights=dw, scales=ds)[over]
+        if int8:
+            dev.check(dev.lib.vmlm_hip_gemm_nt_int8(da, dw, ds, c, m, k, k, None))
+        else:
+            dev.check(dev.lib.vmlm_hip_gemm_nt_bf16(da, dw, c, m, k, k, None))
+        out.append(dev.down(c, (m, k), np.uint32))
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("m,k", [(40, 512), (3, 2304), (77, 1001),
+                                 (1500, 2304),   # C beside the int8 rows: more than the scratch
+                                 (1000, 1500)])  # C beside the terms and the padded copy alike
+def test_gemm_noalloc_over_its_own_rows(dev, m, k):
+    rng = np.random.default_rng(m + k)
+    a, w, _, s = direct_case(rng, m, k, k, True)
+    dw, ds, c, da = dev.up(w), dev.up(s), dev.empty(m * k * 4), dev.up(a)
+    f = dev.lib.vmlm_hip_gemm_nt_int8_noalloc
+    dev.check(f(da, dw, ds, c, m, k, k, None))
+    want = dev.down(c, (m, k), np.float32)
+    dev.check(f(da, dw, ds, da, m, k, k, None))
+    got = dev.down(da, (m, k), np.float32)
+    ref = (a.astype(np.float64) @ w.astype(np.float64).T) * s
+    assert_close_rms(want, ref)
+    assert_close_rms(got, ref)
