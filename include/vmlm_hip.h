@@ -214,7 +214,7 @@ int vmlm_attention_decode_split(const float *q, const float *k_new, const float 
 
 /* ================================================================ layer 2
  * Device pointers, asynchronous on `stream`. Same semantics as layer 1.
- * The result of the int8 and bf16 weight GEMMs may lie over their operands (C
+ * The result of the f32, int8 and bf16 weight GEMMs may lie over their operands (C
  * is then formed in the workspace; where the fixed scratch of the noalloc call
  * has no room for it, a row of A under C with a NaN or an infinity comes out
  * NaN, and weights under C are refused with 9 unless they are staged). */

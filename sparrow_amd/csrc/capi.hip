@@ -264,6 +264,11 @@ static int download(void *host, const void *dev, size_t bytes, hipStream_t st) {
 
 static inline size_t round_up(size_t x, size_t m) { return (x + m - 1) / m * m; }
 
+// Whether the bytes [p, p + np) and [q, q + nq) share any.
+static inline bool overlap(const void *p, size_t np, const void *q, size_t nq) {
+    return (uintptr_t)p < (uintptr_t)q + nq && (uintptr_t)q < (uintptr_t)p + np;
+}
+
 // Whether the one-launch GEMM over the caller's own rows (launch_gemm_direct)
 // is the faster way, against the times of the other paths (us, measured):
 //  * unpadded bf16 at m <= 16: the per-tile GEMV holds up to five rows' (term,
@@ -511,11 +516,9 @@ static int q_matmul(const float *a, const void *W, bool wi8, const float *scale,
                     size_t m, size_t n, size_t k, hipStream_t st, WS &stg,
                     const void *Wsw = nullptr) {
     if (m == 0 || n == 0) return VMLM_OK;
-    auto over = [&](const void *x, size_t bytes) {
-        return (uintptr_t)c < (uintptr_t)x + bytes && (uintptr_t)x < (uintptr_t)c + m * n * 4;
-    };
-    const QOver o{over(a, m * k * 4), over(W, n * k * (wi8 ? 1 : 2))};
-    const bool os = scale && over(scale, n * 4);
+    const size_t cb = m * n * 4;
+    const QOver o{overlap(c, cb, a, m * k * 4), overlap(c, cb, W, n * k * (wi8 ? 1 : 2))};
+    const bool os = scale && overlap(c, cb, scale, n * 4);
     if (!o.a && !o.w && !os) return q_matmul_to(a, W, wi8, scale, c, m, n, k, st, stg, Wsw);
     auto beside = [&]() {
         float *t = stg.template alloc<float>(m * n);
@@ -767,10 +770,11 @@ int vmlm_hip_gemm_nt_bf16bf16(const uint16_t *a, const uint16_t *b, float *c, si
 static int dev_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n, size_t k,
                         bool acc, bool nt, hipStream_t st) {
     Stage stg(st);
-    const size_t wf = gemm_f32_work_floats(m, n, k);
+    const bool over = overlap(c, m * n * 4, a, m * k * 4) || overlap(c, m * n * 4, b, n * k * 4);
+    const size_t wf = gemm_f32_work_floats(m, n, k, over);
     float *work = wf ? stg.alloc<float>(wf) : nullptr;
     STAGE_OK(stg);
-    return launch_gemm_f32(a, b, c, m, n, k, acc, nt, st, work);
+    return launch_gemm_f32(a, b, c, m, n, k, acc, nt, st, work, over);
 }
 int vmlm_hip_gemm_nt(const float *a, const float *b, float *c, size_t m, size_t n, size_t k,
                      bool acc, void *stream) {

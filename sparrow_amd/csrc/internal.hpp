@@ -377,9 +377,11 @@ inline size_t gemm_i8_work_floats(int M, int N, int K) {
 
 // f32 GEMMs (NT and NN) with optional accumulate (k_gemm32.hip).
 // work: gemm_f32_work_floats() floats (small grids are split over k; null: no split).
+// over: c lies over a or b.
 int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n, size_t k,
-                    bool acc, bool b_is_nt, hipStream_t st, float *work = nullptr);
-size_t gemm_f32_work_floats(size_t m, size_t n, size_t k);
+                    bool acc, bool b_is_nt, hipStream_t st, float *work = nullptr,
+                    bool over = false);
+size_t gemm_f32_work_floats(size_t m, size_t n, size_t k, bool over = false);
 
 // Row / elementwise ops.
 int launch_rmsnorm(float *dst, const float *src, const float *g, size_t rows, size_t cols,

@@ -27,6 +27,8 @@
 // steps per tile (to spread the L2 channels of rows 9 KiB apart) changed nothing. A grid of few tiles
 // is split over k (grid z): each slice writes its partial tile to `part`
 // [ks][m][n] and gemm_f32_reduce_kernel sums the slices in order (deterministic).
+// A result over its own operands goes that way with one slice too: the product
+// stores nothing over rows that another tile still reads.
 #include "internal.hpp"
 
 namespace vmlm {
@@ -303,13 +305,13 @@ int launch_shape(const G32Params &p, const Shape &s, hipStream_t st) {
 
 }  // namespace
 
-size_t gemm_f32_work_floats(size_t m, size_t n, size_t k) {
+size_t gemm_f32_work_floats(size_t m, size_t n, size_t k, bool over) {
     const int ks = pick_shape(m, n, k).ks;
-    return ks > 1 ? (size_t)ks * m * n : 0;
+    return ks > 1 || over ? (size_t)ks * m * n : 0;
 }
 
 int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n, size_t k,
-                    bool acc, bool b_is_nt, hipStream_t st, float *work) {
+                    bool acc, bool b_is_nt, hipStream_t st, float *work, bool over) {
     if (m == 0 || n == 0) return VMLM_OK;
     if (k == 0) {
         if (!acc) return launch_fill_zero(c, m * n * sizeof(float), st);
@@ -317,6 +319,7 @@ int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n
     }
     VMLM_GUARD(m <= 0x7fffffffu && n <= 0x7fffffffu && k <= 0x7fffffc0u,
                "gemm f32: shape too large");
+    VMLM_GUARD(work || !over, "gemm f32: a result over its operands needs the workspace");
     Shape s = pick_shape(m, n, k);
     if (!work) s.ks = 1;
     const size_t steps = (k + 63) / 64;
@@ -330,7 +333,7 @@ int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n
     p.acc = acc ? 1 : 0;
     p.kslice = (int)((steps + s.ks - 1) / s.ks * 64);
     s.ks = (int)((k + p.kslice - 1) / p.kslice);
-    p.part = s.ks > 1 ? work : nullptr;
+    p.part = s.ks > 1 || over ? work : nullptr;
     p.group = s.ks > 1 ? 0 : 8;
     const bool vec = k % 4 == 0 && (b_is_nt || n % 4 == 0) && ((uintptr_t)a & 15) == 0 &&
                      ((uintptr_t)b & 15) == 0;

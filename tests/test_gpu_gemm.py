@@ -375,3 +375,33 @@ def test_gemm_noalloc_over_its_own_rows(dev, m, k):
     ref = (a.astype(np.float64) @ w.astype(np.float64).T) * s
     assert_close_rms(want, ref)
     assert_close_rms(got, ref)
+
+
+# f32: no slice at any k, one and more slices otherwise; each tile
+@pytest.mark.parametrize("m,k", [(20, 64), (100, 256), (256, 448), (64, 1030), (1000, 300),
+                                 (1500, 1028), (2100, 96)])
+@pytest.mark.parametrize("over", ["a", "b"])
+def test_gemm_f32_over_its_operands(dev, m, k, over):
+    """n = k, NT and NN, overwriting and accumulating: as in a buffer of its own
+    that held the operand's values."""
+    rng = np.random.default_rng(m + 3 * k)
+    a = rng.standard_normal((m, k), dtype=np.float32)
+    b = rng.standard_normal((k, k), dtype=np.float32)
+    size = max(m, k) * k * 4
+    under = a if over == "a" else b  # what C holds before, where it accumulates
+
+    def put(x):
+        p = dev.empty(size)
+        dev.check(dev.lib.vmlm_hip_memset(p, 0, size))
+        dev.check(dev.lib.vmlm_hip_memcpy_h2d(p, x.ctypes.data, x.nbytes))
+        return p
+
+    for f in (dev.lib.vmlm_hip_gemm_nt, dev.lib.vmlm_hip_gemm):
+        for acc in (False, True):
+            out = []
+            for own in (True, False):
+                da, db = put(a), put(b)
+                c = put(under) if own else da if over == "a" else db
+                dev.check(f(da, db, c, m, k, k, acc, None))
+                out.append(dev.down(c, (m, k), np.uint32))
+            assert np.array_equal(out[0], out[1])
