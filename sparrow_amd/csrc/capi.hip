@@ -613,8 +613,13 @@ int vmlm_hip_memcpy_d2d(void *dst, const void *src, size_t bytes) {
 }
 int vmlm_hip_memset(void *dptr, int value, size_t bytes) {
     INIT_OR_RETURN();
-    // hipMemset may return before the memory is set, and it runs on the legacy
-    // stream, which the library's non-blocking stream does not wait for
+    // hipMemset runs on the legacy stream, which neither waits for the
+    // library's non-blocking stream nor is waited for by it, and may return
+    // before the memory is set: after what the library stream was given (a
+    // stream under capture is given nothing), and before what it is given next
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    VMLM_HIP_CHECK(hipStreamIsCapturing(lib_stream(), &cs));
+    if (cs == hipStreamCaptureStatusNone) VMLM_HIP_CHECK(hipStreamSynchronize(lib_stream()));
     VMLM_HIP_CHECK(hipMemset(dptr, value, bytes));
     VMLM_HIP_CHECK(hipStreamSynchronize(nullptr));
     return VMLM_OK;

@@ -405,3 +405,21 @@ def test_gemm_f32_over_its_operands(dev, m, k, over):
                 dev.check(f(da, db, c, m, k, k, acc, None))
                 out.append(dev.down(c, (m, k), np.uint32))
             assert np.array_equal(out[0], out[1])
+
+
+def test_memset_after_queued_work(dev):
+    """memset comes after the calls that the library stream was given before it
+    (a millisecond of products that write the buffer) and before the next one."""
+    n = 2048
+    rng = np.random.default_rng(4)
+    a = rng.standard_normal((n, n), dtype=np.float32)
+    da, c = dev.up(a), dev.empty(n * n * 4)
+    for _ in range(3):
+        for _ in range(8):
+            dev.check(dev.lib.vmlm_hip_gemm_nt(da, da, c, n, n, n, False, None))
+        dev.check(dev.lib.vmlm_hip_memset(c, 0, n * n * 4))
+        assert not dev.down(c, (n, n), np.uint32).any()
+        dev.check(dev.lib.vmlm_hip_memset(c, 0x3f, n * n * 4))
+        dev.check(dev.lib.vmlm_hip_scale(c, c, n * n, 2.0, None))
+        got = dev.down(c, (n, n), np.float32)
+        assert (got == 2 * np.uint32(0x3f3f3f3f).view(np.float32)).all()
