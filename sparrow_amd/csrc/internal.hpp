@@ -9,6 +9,15 @@ namespace vmlm {
 // constant -2/hd * ln_f(theta), computed once per launch.
 float host_ln_f(float x);
 
+// Lets a kernel have up to `bytes` (the most that any call of it takes) of
+// dynamic LDS. Set before each launch: it belongs to the current device, and an
+// error is of this call.
+inline int allow_lds(const void *kernel, size_t bytes) {
+    VMLM_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)bytes));
+    return VMLM_OK;
+}
+
 // The (N-block, M-block) tile of this workgroup. Workgroups are dispatched
 // round-robin over the 8 XCDs (workgroup i on XCD i % 8), each with its own
 // L2. With `group` > 0 (and the tile count a multiple of 8), XCD x takes the

@@ -540,6 +540,7 @@ static int build_rev(const uint32_t *src, const float *w, size_t E, size_t k0, s
     r.pairs = (uint2 *)take(E * 8 + 8);
     r.off = (uint32_t *)take((d + 1) * 4);
     if (rev_counts(E, d)) {
+        int rc;
         const size_t tiles = rev_tiles(E), d4 = rev_d4(d);
         uint16_t *rank = (uint16_t *)take(E * 2);
         uint16_t *cnt = (uint16_t *)take(tiles * d4 * 2);
@@ -547,10 +548,7 @@ static int build_rev(const uint32_t *src, const float *w, size_t E, size_t k0, s
         uint32_t *tot = (uint32_t *)take(d4 * 4);
         int bits = 0;
         while (((size_t)1 << bits) < d) ++bits;
-        static const hipError_t attr = hipFuncSetAttribute(
-            (const void *)b1_rev_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-            (int)(16 * REV_DMAX));
-        VMLM_HIP_CHECK(attr);
+        if ((rc = allow_lds((const void *)b1_rev_count_kernel, 16 * REV_DMAX))) return rc;
         b1_rev_count_kernel<<<tiles, REV_TILE, 16 * d4, st>>>(src, (uint32_t)E, (int)d, (int)d4,
                                                               bits, rank, cnt);
         VMLM_HIP_CHECK(hipGetLastError());
@@ -602,10 +600,8 @@ int launch_b1_backward(const float *w, const float *srcf, const uint32_t *src, s
 template <int TB>
 static int launch_t8_dx_lds(const RevIndex &r, const float *dyt, size_t t8, size_t d, float *dxt,
                             hipStream_t st) {
-    static const hipError_t attr = hipFuncSetAttribute(
-        (const void *)b1_bwd_t8_dx_lds_kernel<TB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-        (int)B1_DX_LDS);
-    VMLM_HIP_CHECK(attr);
+    const int rc = allow_lds((const void *)b1_bwd_t8_dx_lds_kernel<TB>, B1_DX_LDS);
+    if (rc) return rc;
     const size_t blocks = (t8 + TB - 1) / TB, pass = B1_DX_THREADS / (TB / 4);
     const size_t passes = (d + pass - 1) / pass;
     size_t shares = blocks >= 256 ? 1 : 256 / blocks;

@@ -1,4 +1,4 @@
-"""CPU check of the built kernels' copies from global memory into LDS, which are
+"""CPU checks of LDS use. The copies from global memory into LDS are
 inline assembly (csrc/common.hpp): the wait states that the hardware asks of
 software before such a load are in the code of every kernel that has one. The
 compiler fills them in for its own instructions, not inside an assembly string."""
@@ -82,3 +82,14 @@ def test_lds_copies_have_their_wait_states(tmp_path):
             recent = recent[-7:] + [ins]
     assert loads > 0
     assert not bad, sorted(bad)[:8]
+
+
+def test_lds_sizes_are_set_for_each_launch():
+    """A kernel's dynamic LDS limit belongs to the current device: no launch keeps
+    it, or an error of setting it, from another."""
+    import sparrow_amd
+    from pathlib import Path
+    src = "".join(p.read_text() for p in Path(sparrow_amd.__file__).parent.glob("csrc/*.h*"))
+    assert src.count("hipFuncSetAttribute") == 1  # allow_lds
+    assert src.count("allow_lds(") >= 5
+    assert not re.search(r"\bstatic\b[^;{(]*=\s*(hip|allow_lds)", src)
