@@ -58,7 +58,8 @@ struct G32Params {
     int m, n, k, acc, kslice, group;
 };
 
-template <bool NT, bool VEC, int BM, int BN>
+// NA accumulators a tile: MFMA s of a step adds to accumulator s % NA.
+template <bool NT, bool VEC, int BM, int BN, int NA>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
     constexpr int KS = g32_k<BM, BN>(), ROW = KS * 4, PK = KS / 4;  // pieces of a row along k
     constexpr int A_BYTES = BM * ROW, B_BYTES = BN * ROW, STAGE = A_BYTES + B_BYTES;
@@ -160,11 +161,13 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
         for (int q = 0; q < B_INS; ++q) *(f32x4 *)(sb + A_BYTES + q * 4096) = rb[q];
     };
 
-    f32x4 acc[TM][TN];
+    f32x4 acc[NA][TM][TN];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int n = 0; n < NA; ++n)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[n][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     auto compute = [&](const uint8_t *sA) {
         const uint8_t *sB = sA + A_BYTES;
 #pragma unroll
@@ -192,9 +195,10 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e],
-                                                                         acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < TN; ++j) {
+                        f32x4 &c = acc[(4 * h + e) % NA][i][j];
+                        c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], b[j][e], c, 0, 0, 0);
+                    }
         }
     };
     if constexpr (VEC) issue(0);
@@ -215,6 +219,10 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
+#pragma unroll
+            for (int w = 1; w < NA; w *= 2)
+#pragma unroll
+                for (int n = 0; n < NA; n += 2 * w) acc[n][i][j] = acc[n][i][j] + acc[n + w][i][j];
             const int col = n0 + wn * WN + 16 * j + r;
             if (col >= p.n) continue;
 #pragma unroll
@@ -222,28 +230,35 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
                 const int row = m0 + wm * WM + 16 * i + 4 * g + e;
                 if (row >= p.m) continue;
                 if (p.part) {
-                    p.part[((size_t)blockIdx.z * p.m + row) * p.n + col] = acc[i][j][e];
+                    p.part[((size_t)blockIdx.z * p.m + row) * p.n + col] = acc[0][i][j][e];
                 } else {
                     float *o = p.C + (size_t)row * p.n + col;
-                    *o = p.acc ? *o + acc[i][j][e] : acc[i][j][e];
+                    *o = p.acc ? *o + acc[0][i][j][e] : acc[0][i][j][e];
                 }
             }
         }
 }
 
-constexpr int G32_SLICES = 16;
 __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const float *__restrict__ part,
                                                               int ks, size_t mn,
                                                               float *__restrict__ C, int acc) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= mn) return;
-    float v[G32_SLICES];  // every slice in flight, then summed in order
+    // 16 slices in flight, then summed in order
+    float v[16];
 #pragma unroll
-    for (int z = 0; z < G32_SLICES; ++z) v[z] = part[(size_t)(z < ks ? z : ks - 1) * mn + i];
+    for (int z = 0; z < 16; ++z) v[z] = part[(size_t)(z < ks ? z : ks - 1) * mn + i];
     float sum = v[0];
 #pragma unroll
-    for (int z = 1; z < G32_SLICES; ++z)
+    for (int z = 1; z < 16; ++z)
         if (z < ks) sum += v[z];
+    for (int z0 = 16; z0 < ks; z0 += 16) {
+#pragma unroll
+        for (int z = 0; z < 16; ++z) v[z] = part[(size_t)(z0 + z < ks ? z0 + z : ks - 1) * mn + i];
+#pragma unroll
+        for (int z = 0; z < 16; ++z)
+            if (z0 + z < ks) sum += v[z];
+    }
     C[i] = acc ? C[i] + sum : sum;
 }
 
@@ -251,9 +266,11 @@ __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const float *__res
 // copies per product (128 x 128: 129 TFLOP/s at 4096^3; 64 x 64 119, 32 x 64 107,
 // 32 x 32 102), `one` what it loses alone on its CU (fewer accumulators to keep
 // a matrix core busy). Then the k-slices, of 128 at least, that give a small
-// grid about two workgroups per CU (the second launch costs about five steps).
+// grid about two workgroups per CU (the second launch costs about five steps):
+// 16 at most, from k = 16384 on one per 1024 of k and 64 at most (32 x 32 x 65536:
+// 37 us with 16, 14.6 with 64).
 struct Shape {
-    int bm, bn, ks;
+    int bm, bn, ks, sums;
 };
 Shape pick_tile(size_t m, size_t n) {
     struct Tile {
@@ -262,7 +279,7 @@ Shape pick_tile(size_t m, size_t n) {
     };
     constexpr Tile tiles[] = {{128, 128, 1.0, 1.0}, {64, 64, 1.08, 1.1}, {32, 64, 1.17, 1.15},
                               {32, 32, 1.26, 1.0}};
-    Shape best{32, 32, 1};
+    Shape best{32, 32, 1, 1};
     if ((size_t)cdiv(m, 32) * cdiv(n, 32) <= 256) return best;  // one round of the smallest
     double least = 1e300;
     for (const Tile &t : tiles) {
@@ -282,16 +299,22 @@ Shape pick_shape(size_t m, size_t n, size_t k) {
     if (wgs <= 128 && steps >= 8) {
         size_t ks = 512 / wgs;
         if (ks > steps / 2) ks = steps / 2;
-        if (ks > G32_SLICES) ks = G32_SLICES;
+        const size_t most = steps <= 256 ? 16 : steps / 16 < 64 ? steps / 16 : 64;
+        if (ks > most) ks = most;
         best.ks = (int)ks;
     }
+    // fewer than 128 tiles: eight accumulators, so that a run of k is no longer
+    // for it than in slices of 64 (100 x 256 x 448, one slice: relative error
+    // 3.8e-7 with one, 1.9e-7 with four, 1.4e-7 with eight; 0.1 us; 32 x 32 x
+    // 65536 1.1e-6 with one and 16 slices, 4.0e-7 in 256, now 2.5e-7)
+    if ((size_t)cdiv(m, 32) * cdiv(n, 32) < 128 && k >= 128) best.sums = 8;
     return best;
 }
 
-template <bool NT, bool VEC, int BM, int BN>
+template <bool NT, bool VEC, int BM, int BN, int NA = 1>
 int launch_tile(const G32Params &p, int ks, hipStream_t st) {
     const dim3 grid(cdiv((size_t)p.n, BN), cdiv((size_t)p.m, BM), ks);
-    gemm_f32_kernel<NT, VEC, BM, BN><<<grid, 256, 0, st>>>(p);
+    gemm_f32_kernel<NT, VEC, BM, BN, NA><<<grid, 256, 0, st>>>(p);
     VMLM_HIP_CHECK(hipGetLastError());
     return VMLM_OK;
 }
@@ -300,6 +323,7 @@ int launch_shape(const G32Params &p, const Shape &s, hipStream_t st) {
     if (s.bm == 128) return launch_tile<NT, VEC, 128, 128>(p, s.ks, st);
     if (s.bm == 64) return launch_tile<NT, VEC, 64, 64>(p, s.ks, st);
     if (s.bn == 64) return launch_tile<NT, VEC, 32, 64>(p, s.ks, st);
+    if (s.sums > 1) return launch_tile<NT, VEC, 32, 32, 8>(p, s.ks, st);
     return launch_tile<NT, VEC, 32, 32>(p, s.ks, st);
 }
 

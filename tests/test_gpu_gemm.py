@@ -423,3 +423,21 @@ def test_memset_after_queued_work(dev):
         dev.check(dev.lib.vmlm_hip_scale(c, c, n * n, 2.0, None))
         got = dev.down(c, (n, n), np.float32)
         assert (got == 2 * np.uint32(0x3f3f3f3f).view(np.float32)).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(m, n, k) for m, n in [(1, 40), (33, 64), (100, 256)]
+                                   for k in (130, 448, 2304, 16384, 65536) if m * k < 6e6])
+def test_gemm_f32_sums_in_short_runs(dev, m, n, k):
+    """Outputs of few tiles: 1 + (k - 1) 2^-25. A product that meets a sum with the
+    1 in it is lost, so the error counts the products of that sum's run (at most
+    64, or 128 past k = 2304), and half an ulp of 1 for each sum of runs (eight
+    accumulators, in three steps) and of slices (64 at most)."""
+    a = np.full((m, k), 2.0 ** -25, np.float32)
+    a[:, 0] = 1
+    c = dev.empty(m * n * 4)
+    da, db = dev.up(a), dev.up(np.ones((n, k), np.float32))
+    run, slices = 64 if k <= 2304 else 128, 1 if k < 449 else 64
+    for f in (dev.lib.vmlm_hip_gemm_nt, dev.lib.vmlm_hip_gemm):  # ones either way
+        dev.check(f(da, db, c, m, n, k, False, None))
+        got = dev.down(c, (m, n), np.float32).astype(np.float64)
+        assert np.abs(got - (1 + (k - 1) * 2.0 ** -25)).max() <= (run + 2 * (3 + slices)) * 2.0 ** -25
