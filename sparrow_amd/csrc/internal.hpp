@@ -18,28 +18,6 @@ inline int allow_lds(const void *kernel, size_t bytes) {
     return VMLM_OK;
 }
 
-// The (N-block, M-block) tile of this workgroup. Workgroups are dispatched
-// round-robin over the 8 XCDs (workgroup i on XCD i % 8), each with its own
-// L2. With `group` > 0 (and the tile count a multiple of 8), XCD x takes the
-// x-th eighth of the tiles in a grouped order -- `group` M-blocks at a time,
-// N-blocks walked inside the group -- so the workgroups resident on one XCD
-// at once share A rows and W rows through its L2. A bijection on the tiles.
-__device__ __forceinline__ void gemm_tile(int group, int &bx, int &by) {
-    const int nbx = (int)gridDim.x, nby = (int)gridDim.y, n = nbx * nby;
-    int id = (int)blockIdx.y * nbx + (int)blockIdx.x;
-    if (group <= 0) {
-        bx = (int)blockIdx.x;
-        by = (int)blockIdx.y;
-        return;
-    }
-    if (n % 8 == 0) id = (id % 8) * (n / 8) + id / 8;
-    const int per = group * nbx;
-    const int m0 = id / per * group, r = id % per;
-    const int gm = nby - m0 < group ? nby - m0 : group;
-    by = m0 + r % gm;
-    bx = r / gm;
-}
-
 // Activation operand of the MFMA GEMV / GEMM: T planes of bf16 bits
 // [T][rows][ld] (ld a multiple of 64, zero padded) whose sum is the f32
 // activation (see split_bf16).

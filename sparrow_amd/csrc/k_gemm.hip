@@ -31,6 +31,28 @@ struct GemmI8Params : GemmParams {
     NonfiniteRows nf;  // rows with a NaN factor (GemmArgs)
 };
 
+// The (N-block, M-block) tile of this workgroup. Workgroups are dispatched
+// round-robin over the 8 XCDs (workgroup i on XCD i % 8), each with its own
+// L2. With `group` > 0 (and the tile count a multiple of 8), XCD x takes the
+// x-th eighth of the tiles in a grouped order -- `group` M-blocks at a time,
+// N-blocks walked inside the group -- so the workgroups resident on one XCD
+// at once share A rows and W rows through its L2. A bijection on the tiles.
+__device__ __forceinline__ void gemm_tile(int group, int &bx, int &by) {
+    const int nbx = (int)gridDim.x, nby = (int)gridDim.y, n = nbx * nby;
+    int id = (int)blockIdx.y * nbx + (int)blockIdx.x;
+    if (group <= 0) {
+        bx = (int)blockIdx.x;
+        by = (int)blockIdx.y;
+        return;
+    }
+    if (n % 8 == 0) id = (id % 8) * (n / 8) + id / 8;
+    const int per = group * nbx;
+    const int m0 = id / per * group, r = id % per;
+    const int gm = nby - m0 < group ? nby - m0 : group;
+    by = m0 + r % gm;
+    bx = r / gm;
+}
+
 typedef __attribute__((__vector_size__(4 * sizeof(int)))) int gi32x4;
 
 __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {

@@ -22,13 +22,17 @@
 // The MFMA rate bounds large shapes (a 16 x 16 x 4 product takes a matrix core 32
 // cycles; the clock settles near 2.1 GHz under them), so the tile is chosen for an
 // even load of the CUs. Against a register-staged kernel of 32 x 32 tiles: 1000 x
-// 2304 x 2304 NT 125 -> 113 us, 2048^3 176 -> 140 (123 TFLOP/s), 4096^3 1400 ->
-// 1045, 1500 x 1537 x 1535 (rows off 16 bytes) 193 -> 88. A rotated order of the
-// steps per tile (to spread the L2 channels of rows 9 KiB apart) changed nothing. A grid of few tiles
-// is split over k (grid z): each slice writes its partial tile to `part`
-// [ks][m][n] and gemm_f32_reduce_kernel sums the slices in order (deterministic).
-// A result over its own operands goes that way with one slice too: the product
-// stores nothing over rows that another tile still reads.
+// 2304 x 2304 NT 125 -> 105 us, 2048^3 176 -> 141 (122 TFLOP/s), 4096^3 1400 ->
+// 1030, 1500 x 1537 x 1535 (rows off 16 bytes) 193 -> 88. A rotated order of the
+// steps per tile (to spread the L2 channels of rows 9 KiB apart) changed nothing,
+// and tiles in an order that shares an XCD's L2 neither (4096^3 1030 us with
+// both). The divisions of that order, an address loaded before the first copy and
+// LDS for two stages where there is one step cost a short k up to 0.8 us (500 x
+// 2304 x 64 5.4 us with them, 4.6 without; 161 x 1536 x 64 NN 3.6 and 3.0). A grid
+// of few tiles is split over k (grid z): each slice writes its partial tile to
+// `part` [ks][m][n] and gemm_f32_reduce_kernel sums the slices in order
+// (deterministic). A result over its own operands goes that way with one slice
+// too: the product stores nothing over rows that another tile still reads.
 #include "internal.hpp"
 
 namespace vmlm {
@@ -55,7 +59,7 @@ __device__ __forceinline__ int nn_row(int k) {
 struct G32Params {
     const float *A, *B;
     float *C, *part;
-    int m, n, k, acc, kslice, group;
+    int m, n, k, acc, kslice;
 };
 
 // NA accumulators a tile: MFMA s of a step adds to accumulator s % NA.
@@ -66,14 +70,12 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
     constexpr int A_INS = A_BYTES / 4096, B_INS = B_BYTES / 4096;  // pieces a lane copies a step
     constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
     static_assert(A_INS >= 1 && B_INS >= 1 && TM >= 1 && TN >= 1, "tile too small");
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * STAGE];
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];  // two stages, or the only step's
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, g = lane >> 4, r = lane & 15;
-    int tbx, tby;
-    gemm_tile(p.group, tbx, tby);
-    const int m0 = tby * BM, n0 = tbx * BN;
+    const int m0 = (int)blockIdx.y * BM, n0 = (int)blockIdx.x * BN;
     const int kb = (int)blockIdx.z * p.kslice;
     const int ke = kb + p.kslice < p.k ? kb + p.kslice : p.k;
     const int nk = (ke - kb + KS - 1) / KS;
@@ -114,16 +116,18 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
     const size_t bstep = NT ? KS : (size_t)KS * p.n;
     auto issue = [&](int kt) {  // rows of whole 16-byte pieces, straight into LDS
         const uint32_t sb = lds0 + (uint32_t)((kt & 1) * STAGE);
-        const bool tail = kb + (kt + 1) * KS > ke;
-        auto copy = [&](const float *src, int kin, uint32_t dst) {
-            if (tail && kb + kt * KS + kin >= ke) src = g32_zero;
-            dma16(src, dst);
+        auto copies = [&](auto piece) {
+#pragma unroll
+            for (int q = 0; q < A_INS; ++q)
+                dma16(piece(as[q] + kt * KS, ak[q]), sb + (q * 4 + wave) * 1024);
+#pragma unroll
+            for (int q = 0; q < B_INS; ++q)
+                dma16(piece(bs[q] + kt * bstep, bk[q]), sb + A_BYTES + (q * 4 + wave) * 1024);
         };
-#pragma unroll
-        for (int q = 0; q < A_INS; ++q) copy(as[q] + kt * KS, ak[q], sb + (q * 4 + wave) * 1024);
-#pragma unroll
-        for (int q = 0; q < B_INS; ++q)
-            copy(bs[q] + kt * bstep, bk[q], sb + A_BYTES + (q * 4 + wave) * 1024);
+        const int left = ke - (kb + kt * KS);
+        // (apart, so that a whole step does not wait for the zero's address)
+        if (left >= KS) copies([](const float *src, int) { return src; });
+        else copies([&](const float *src, int k) { return k < left ? src : g32_zero; });
     };
     // rows at any float: the pieces through registers, those that cross the end
     // of a row (the last step, an NN B's last columns) element by element
@@ -215,6 +219,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
         compute(smem + (kt & 1) * STAGE);
     }
 
+    float *out = p.part ? p.part + (size_t)blockIdx.z * p.m * p.n : p.C;
+    const bool add = p.acc && !p.part;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -223,18 +229,13 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(G32Params p) {
             for (int w = 1; w < NA; w *= 2)
 #pragma unroll
                 for (int n = 0; n < NA; n += 2 * w) acc[n][i][j] = acc[n][i][j] + acc[n + w][i][j];
-            const int col = n0 + wn * WN + 16 * j + r;
+            const int col = n0 + wn * WN + 16 * j + r, row = m0 + wm * WM + 16 * i + 4 * g;
             if (col >= p.n) continue;
+            float *o = out + (size_t)row * p.n + col;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int row = m0 + wm * WM + 16 * i + 4 * g + e;
-                if (row >= p.m) continue;
-                if (p.part) {
-                    p.part[((size_t)blockIdx.z * p.m + row) * p.n + col] = acc[0][i][j][e];
-                } else {
-                    float *o = p.C + (size_t)row * p.n + col;
-                    *o = p.acc ? *o + acc[0][i][j][e] : acc[0][i][j][e];
-                }
+                if (row + e >= p.m) continue;
+                o[(size_t)e * p.n] = add ? o[(size_t)e * p.n] + acc[0][i][j][e] : acc[0][i][j][e];
             }
         }
 }
@@ -266,7 +267,9 @@ __global__ __launch_bounds__(256) void gemm_f32_reduce_kernel(const float *__res
 // copies per product (128 x 128: 129 TFLOP/s at 4096^3; 64 x 64 119, 32 x 64 107,
 // 32 x 32 102), `one` what it loses alone on its CU (fewer accumulators to keep
 // a matrix core busy). Then the k-slices, of 128 at least, that give a small
-// grid about two workgroups per CU (the second launch costs about five steps):
+// grid about two workgroups per CU (the second launch costs six steps, eight
+// where it reduces more: 32 x 256 x 448 6.2 -> 6.0 us, 64 x 1024 x 448 6.2 -> 6.5, 114 x
+// 768 x 512 6.8 -> 7.0):
 // 16 at most, from k = 16384 on one per 1024 of k and 64 at most (32 x 32 x 65536:
 // 37 us with 16, 14.6 with 64).
 struct Shape {
@@ -296,7 +299,7 @@ Shape pick_tile(size_t m, size_t n) {
 Shape pick_shape(size_t m, size_t n, size_t k) {
     Shape best = pick_tile(m, n);
     const size_t wgs = (size_t)cdiv(m, best.bm) * cdiv(n, best.bn), steps = (k + 63) / 64;
-    if (wgs <= 128 && steps >= 8) {
+    if (wgs <= 128 && steps >= (wgs > 64 ? 10 : wgs > 32 ? 8 : 7)) {
         size_t ks = 512 / wgs;
         if (ks > steps / 2) ks = steps / 2;
         const size_t most = steps <= 256 ? 16 : steps / 16 < 64 ? steps / 16 : 64;
@@ -314,7 +317,10 @@ Shape pick_shape(size_t m, size_t n, size_t k) {
 template <bool NT, bool VEC, int BM, int BN, int NA = 1>
 int launch_tile(const G32Params &p, int ks, hipStream_t st) {
     const dim3 grid(cdiv((size_t)p.n, BN), cdiv((size_t)p.m, BM), ks);
-    gemm_f32_kernel<NT, VEC, BM, BN, NA><<<grid, 256, 0, st>>>(p);
+    constexpr int KS = g32_k<BM, BN>(), stage = (BM + BN) * KS * 4;
+    static_assert(2 * stage <= 64 * 1024, "");
+    const int lds = (p.kslice < p.k ? p.kslice : p.k) <= KS ? stage : 2 * stage;
+    gemm_f32_kernel<NT, VEC, BM, BN, NA><<<grid, 256, lds, st>>>(p);
     VMLM_HIP_CHECK(hipGetLastError());
     return VMLM_OK;
 }
@@ -358,7 +364,6 @@ int launch_gemm_f32(const float *a, const float *b, float *c, size_t m, size_t n
     p.kslice = (int)((steps + s.ks - 1) / s.ks * 64);
     s.ks = (int)((k + p.kslice - 1) / p.kslice);
     p.part = s.ks > 1 || over ? work : nullptr;
-    p.group = s.ks > 1 ? 0 : 8;
     const bool vec = k % 4 == 0 && (b_is_nt || n % 4 == 0) && ((uintptr_t)a & 15) == 0 &&
                      ((uintptr_t)b & 15) == 0;
     const int rc = b_is_nt ? vec ? launch_shape<true, true>(p, s, st) : launch_shape<true, false>(p, s, st)
