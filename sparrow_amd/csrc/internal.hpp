@@ -9,12 +9,13 @@ namespace vmlm {
 // constant -2/hd * ln_f(theta), computed once per launch.
 float host_ln_f(float x);
 
-// Lets a kernel have up to `bytes` (the most that any call of it takes) of
-// dynamic LDS. Set before each launch: it belongs to the current device, and an
-// error is of this call.
-inline int allow_lds(const void *kernel, size_t bytes) {
-    VMLM_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)bytes));
+// Lets a kernel have `lds` bytes of dynamic LDS (`most`: the most that any call of
+// it takes). Set at each launch that needs more than every kernel may have: it
+// belongs to the current device, and an error is of this call.
+inline int allow_lds(const void *kernel, size_t lds, size_t most) {
+    if (lds > 64 * 1024)
+        VMLM_HIP_CHECK(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)most));
     return VMLM_OK;
 }
 

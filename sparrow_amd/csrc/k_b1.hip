@@ -337,7 +337,7 @@ template <int G>
 static int launch_layer_g(const void *plan, int n, int d, const float *x, size_t xbs, size_t xrs,
                           int n_tokens, float *y, size_t ybs, size_t yrs, int act, hipStream_t st) {
     const size_t lds = (size_t)(((d + 15) & ~15) + 1) * B1_ROW;
-    const int rc = allow_lds((const void *)b1_t8_layer_kernel<G>,
+    const int rc = allow_lds((const void *)b1_t8_layer_kernel<G>, lds,
                              ((B1_DMAX + 15) / 16 * 16 + 1) * B1_ROW);
     if (rc) return rc;
     const uint4 *off = (const uint4 *)plan;
@@ -533,10 +533,10 @@ size_t b1_stack_plan_bytes(int d, const int *k0, int n_layers) {
 template <int G>
 static int launch_stack_g(const char *plan, size_t stride, int n_layers, int d, const float *x,
                           float *y, int T, int act, hipStream_t st) {
-    const int rc = allow_lds((const void *)b1_stack_kernel<G>,
+    const size_t lds = 2 * (size_t)(((d + 15) & ~15) + 1) * B1_SROW;
+    const int rc = allow_lds((const void *)b1_stack_kernel<G>, lds,
                              2 * ((B1_SDMAX + 15) / 16 * 16 + 1) * B1_SROW);
     if (rc) return rc;
-    const size_t lds = 2 * (size_t)(((d + 15) & ~15) + 1) * B1_SROW;
     b1_stack_kernel<G><<<cdiv((size_t)T, 4), 64 * B1_SNW, lds, st>>>(plan, stride, n_layers, d, x,
                                                                       y, T, act);
     VMLM_HIP_CHECK(hipGetLastError());

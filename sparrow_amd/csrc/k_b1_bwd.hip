@@ -548,7 +548,7 @@ static int build_rev(const uint32_t *src, const float *w, size_t E, size_t k0, s
         uint32_t *tot = (uint32_t *)take(d4 * 4);
         int bits = 0;
         while (((size_t)1 << bits) < d) ++bits;
-        if ((rc = allow_lds((const void *)b1_rev_count_kernel, 16 * REV_DMAX))) return rc;
+        if ((rc = allow_lds((const void *)b1_rev_count_kernel, 16 * d4, 16 * REV_DMAX))) return rc;
         b1_rev_count_kernel<<<tiles, REV_TILE, 16 * d4, st>>>(src, (uint32_t)E, (int)d, (int)d4,
                                                               bits, rank, cnt);
         VMLM_HIP_CHECK(hipGetLastError());
@@ -600,7 +600,7 @@ int launch_b1_backward(const float *w, const float *srcf, const uint32_t *src, s
 template <int TB>
 static int launch_t8_dx_lds(const RevIndex &r, const float *dyt, size_t t8, size_t d, float *dxt,
                             hipStream_t st) {
-    const int rc = allow_lds((const void *)b1_bwd_t8_dx_lds_kernel<TB>, B1_DX_LDS);
+    const int rc = allow_lds((const void *)b1_bwd_t8_dx_lds_kernel<TB>, d * TB * 4, B1_DX_LDS);
     if (rc) return rc;
     const size_t blocks = (t8 + TB - 1) / TB, pass = B1_DX_THREADS / (TB / 4);
     const size_t passes = (d + pass - 1) / pass;
