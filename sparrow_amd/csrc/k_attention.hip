@@ -136,7 +136,7 @@ struct PrefillParams {
     int S, Sp, ldo, causal, nqb, H;
     int nseq;
     int o_vec;     // O rows 16-byte aligned: float4 stores
-    float scale2;  // score scale times log2(e)
+    float scale;
 };
 
 // Q, K and V of every (sequence, head) as bf16 term planes, rows padded to Sp
@@ -260,13 +260,18 @@ __global__ __launch_bounds__(1024) void attn_qkv_prep_kernel(QKVPrepParams p) {
 // One key block of the prefill attention for the wave's NQ x 16 queries: S^T =
 // K Q^T over the block's 64 keys (two bf16 terms of K and of Q), the online
 // softmax update of (m, l, o), then O^T += V^T P^T (three terms of V, two of
-// P). T: the block's tile in LDS; lane (g, r) owns queries qa + 16 n. scale2 is
-// the score scale times log2(e): the maximum m and the exponents are in base
-// 2. Only a block that crosses the diagonal or the last key masks.
+// P). T: the block's tile in LDS; lane (g, r) owns queries qa + 16 n. The scores
+// are scaled as OP_SCALE does and log2(e) multiplies their distance from the
+// maximum (att_exp): in the scale, it would round at the score's own magnitude,
+// 2^-10 of a weight at scores of 16000. Only a block that crosses the diagonal or
+// the last key masks.
+__device__ __forceinline__ float att_exp(float x) {
+    return __builtin_amdgcn_exp2f(x * 1.44269504f);
+}
 template <int NQ>
 __device__ __forceinline__ void prefill_block(const uint16_t (*T)[AT_B][AT_B],
                                               const u32x4 (&aq)[NQ][2][2], int k0, int qa, int S,
-                                              int causal, float scale2, float (&m)[NQ],
+                                              int causal, float scale, float (&m)[NQ],
                                               float (&l)[NQ], f32x4 (&o)[NQ][4]) {
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
     // S^T: block j = keys 16j..16j+15; lane (g, r): keys 16j + 4g + i of
@@ -309,13 +314,13 @@ __device__ __forceinline__ void prefill_block(const uint16_t (*T)[AT_B][AT_B],
                 for (int i = 0; i < 4; ++i) {
                     const int ka = k0 + 16 * j + 4 * g + i;
                     const bool valid = ka < S && (!causal || ka <= qa + 16 * n);
-                    sc[n][j][i] = valid ? sc[n][j][i] * scale2 : -INFINITY;
+                    sc[n][j][i] = valid ? sc[n][j][i] * scale : -INFINITY;
                 }
         } else {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) sc[n][j][i] = sc[n][j][i] * scale2;
+                for (int i = 0; i < 4; ++i) sc[n][j][i] = sc[n][j][i] * scale;
         }
         float mx = -INFINITY;
 #pragma unroll
@@ -327,13 +332,13 @@ __device__ __forceinline__ void prefill_block(const uint16_t (*T)[AT_B][AT_B],
         const float mn = fmaxf(m[n], mx);
         // no finite score yet: exponents of -inf - 0 are 0 (not -inf - -inf = NaN)
         const float mref = mn == -INFINITY ? 0.0f : mn;
-        const float alpha = __builtin_amdgcn_exp2f(m[n] - mref);
+        const float alpha = att_exp(m[n] - mref);
         float rs = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                sc[n][j][i] = __builtin_amdgcn_exp2f(sc[n][j][i] - mref);
+                sc[n][j][i] = att_exp(sc[n][j][i] - mref);
                 rs += sc[n][j][i];
             }
         rs += lane_xor16(rs);
@@ -434,7 +439,7 @@ __device__ __forceinline__ bool prefill_unit(int nqb, int H, int nseq, int causa
 // with the first group (the one-launch kernel's sum, the same bits). Each group
 // copies its tiles straight into its two LDS stages, the next one while the
 // current one is consumed. 36 heads, 1000 causal rows, with the
-// prep launch: 83.6 -> 46 us (2048 rows 244 -> 125).
+// prep launch: 83.6 -> 47 us (2048 rows 244 -> 127).
 constexpr int AT_SPLIT = 4;
 template <int NQ, int NG>
 __global__ __launch_bounds__(256 * NG, 2) void attn_prefill_kernel(PrefillParams P) {
@@ -492,7 +497,7 @@ __global__ __launch_bounds__(256 * NG, 2) void attn_prefill_kernel(PrefillParams
         if (kb + st < end) issue(kb + st, stage ^ 1);
         // (a wave whose queries all lie above the block skips it)
         if (kb < end && (!causal || kb * AT_B <= q0 + 16 * NQ - 1))
-            prefill_block<NQ>(tiles[grp][stage], aq, kb * AT_B, qa, S, causal, P.scale2, m, l, o);
+            prefill_block<NQ>(tiles[grp][stage], aq, kb * AT_B, qa, S, causal, P.scale, m, l, o);
         stage ^= 1;
     }
     if (NG == 2 && st == 2) {
@@ -514,8 +519,8 @@ __global__ __launch_bounds__(256 * NG, 2) void attn_prefill_kernel(PrefillParams
             for (int n = 0; n < NQ; ++n) {
                 const float m1 = x[(18 * n) * 256 + tid], l1 = x[(18 * n + 1) * 256 + tid];
                 const float mt = fmaxf(m[n], m1), mref = mt == -INFINITY ? 0.0f : mt;
-                const float a0 = __builtin_amdgcn_exp2f(m[n] - mref);
-                const float a1 = __builtin_amdgcn_exp2f(m1 - mref);
+                const float a0 = att_exp(m[n] - mref);
+                const float a1 = att_exp(m1 - mref);
                 l[n] = l[n] * a0 + l1 * a1;
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
@@ -545,7 +550,7 @@ struct QKVPrefillParams {
     float *kc, *vc;          // KV cache [sequence][head][hs][64], or null
     size_t sin, sout;
     int S, ld, ldo, causal, nqb, H, nseq, hs, rope, o_vec;
-    float scale2, rope_step, pos0;
+    float scale, rope_step, pos0;
     const float2 *tab;       // (sin, cos) of [row][pair index], or null
 };
 
@@ -708,7 +713,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_qkv_kernel(QKVPrefillPara
         __syncthreads();
         if (kb + 1 < kb1) load_kv(kb + 1);
         __builtin_amdgcn_sched_barrier(0);
-        prefill_block<1>(T, aq, kb * AT_B, qa, S, causal, P.scale2, m, l, o);
+        prefill_block<1>(T, aq, kb * AT_B, qa, S, causal, P.scale, m, l, o);
     }
     prefill_store(o[0], l[0], qa, S, P.O, P.sout, P.ldo, P.o_vec, h, z);
 }
@@ -755,7 +760,6 @@ int launch_attention_prefill(const float *q, const float *k, const float *v, flo
     VMLM_GUARD(nseq >= 1 && nseq <= 65535 && H <= 65535, "attention prefill: grid too large");
     if (S <= 0) return VMLM_OK;
     const int Sp = (S + AT_B - 1) / AT_B * AT_B;
-    const float scale2 = (float)((double)scale * 1.4426950408889634);
     VMLM_GUARD((long long)H * nseq <= 1 << 24 && prefill_grid(Sp / AT_B, H * nseq) <= 1 << 30,
                "attention prefill: grid too large");
     // up to four query blocks over a full grid: one launch from the f32 rows
@@ -781,7 +785,7 @@ int launch_attention_prefill(const float *q, const float *k, const float *v, flo
         F.hs = hs;
         F.rope = rope ? 1 : 0;
         F.o_vec = ((uintptr_t)out & 15) == 0 && ldo % 4 == 0 && (nseq == 1 || sout % 4 == 0);
-        F.scale2 = scale2;
+        F.scale = scale;
         F.rope_step = rope_step;
         F.pos0 = pos0;
         F.tab = rope && ((uintptr_t)rope_tab & 15) == 0 ? rope_tab : nullptr;  // 16-byte table loads
@@ -826,7 +830,7 @@ int launch_attention_prefill(const float *q, const float *k, const float *v, flo
     P.H = H;
     P.o_vec = ((uintptr_t)out & 15) == 0 && ldo % 4 == 0 && (nseq == 1 || sout % 4 == 0);
     P.nseq = nseq;
-    P.scale2 = scale2;
+    P.scale = scale;
     // 32 queries a wave once that still gives every CU a workgroup
     const int nq = (long long)((S + 127) / 128) * H * nseq >= 256 ? 2 : 1;
     P.nqb = (S + 64 * nq - 1) / (64 * nq);

@@ -487,6 +487,29 @@ def test_attention_prefill_one_launch_same_bits(ops, oracle):
         assert_close_rms(got, ref)
 
 
+@pytest.mark.parametrize("S,H", [(256, 64), (300, 2)])  # one launch; two
+def test_attention_prefill_large_scores(ops, S, H):
+    """Scores near 16000 that differ by a few: the weights depend on the
+    differences, which the scaled scores hold exactly (integers; the rotation
+    leaves the dims used here as they are at this theta), so they must not be
+    rounded at the scores' own magnitude. The weights' two bf16 terms give
+    2^-17 of a weight, about 4e-6 of the output's RMS at the worst element."""
+    rng = np.random.default_rng(S)
+    q, k = np.zeros((2, S, H, 64), np.float32)
+    dims = np.r_[16:32, 48:64]
+    q[..., dims] = 16
+    k[..., dims] = 250
+    k[..., 16] += rng.integers(0, 4, (S, H))
+    v = rng.standard_normal((S, H, 64), dtype=np.float32)
+    got = ops.attention_prefill(q.reshape(S, -1), k.reshape(S, -1), v.reshape(S, -1), H,
+                                theta=1e30).reshape(S, H, 64)
+    s = np.einsum("qhd,khd->hqk", q.astype(np.float64), k.astype(np.float64)) * 0.125
+    s = np.where(np.tril(np.ones((S, S), bool)), s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = np.einsum("hqk,khd->qhd", p / p.sum(-1, keepdims=True), v.astype(np.float64))
+    assert_close_rms(got, ref, 2e-5)
+
+
 @pytest.mark.parametrize("H,pos", [(36, 1023), (36, 700), (4, 511), (36, 300)])
 def test_attention_decode_cfg2(ops, oracle, H, pos):
     """Config 2 decode: 1 query against a KV cache of length 1024 (pos 1023),
