@@ -301,8 +301,36 @@ static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
     return 1.1 * us < 10.0 + copy + (steps > prod ? steps : prod);
 }
 
+// int8 weights, up to FX_ROWS rows: one full-K launch whose waves split their
+// k-runs of the f32 rows into int8 terms themselves. True if it takes the call;
+// it needs no workspace and is asked first, since a decode step's projection is
+// little more than its launch (1 x 2304 x 2304: 4.4 us).
+static bool q_few_rows(const float *a, const void *W, const float *scale, float *c, size_t m,
+                       size_t n, size_t k, hipStream_t st, const void *Wsw, int *rc) {
+    if (m > FX_ROWS || m == 0 || n == 0 || k == 0 || k % 128 != 0 || k > (size_t)1 << 30 ||
+        (((uintptr_t)W | (uintptr_t)a) & 15) != 0 || !fx_run_blocks((int)k))
+        return false;
+    const size_t cb = m * n * 4;
+    if (overlap(c, cb, a, m * k * 4) || overlap(c, cb, W, n * k) || overlap(c, cb, scale, n * 4))
+        return false;
+    FxArgs x;
+    x.W = Wsw ? Wsw : W;
+    x.swizzled = Wsw != nullptr;
+    x.ldw = (int)k;
+    x.scale = scale;
+    x.X = a;
+    x.ldx = (int)k;
+    x.C = c;
+    x.ldc = (int)n;
+    x.M = (int)m;
+    x.N = (int)n;
+    x.K = (int)k;
+    *rc = launch_fx_gemv(x, st);
+    return true;
+}
+
 // int8 / bf16 weight GEMM on device operands: C[m,n] = A[m,k] . W[n,k]^T (* scale).
-// int8 weights and m <= 16: the full-K GEMV (m <= FX_ROWS) or the wide k-split
+// int8 weights and m <= 16: the full-K GEMV (q_few_rows) or the wide k-split
 // GEMV; where it is faster (q_direct), one launch over the rows as they are;
 // int8 weights, m > 16 and K a multiple of 128, int8 rows and the int8 MFMA
 // GEMM; otherwise A split into 3 bf16 terms, K padded to a multiple of 128,
@@ -320,6 +348,8 @@ template <class WS>
 static int q_matmul_to(const float *a, const void *W, bool wi8, const float *scale, float *c,
                        size_t m, size_t n, size_t k, hipStream_t st, WS &stg, const void *Wsw,
                        QOver over = QOver{}) {
+    int rcf;
+    if (wi8 && q_few_rows(a, W, scale, c, m, n, k, st, Wsw, &rcf)) return rcf;
     const size_t esz = wi8 ? 1 : 2;
     const size_t Kp = round_up(k == 0 ? 1 : k, 128);  // one 128-byte GEMV chunk covers 128 k
     const bool padded = Kp != k || ((uintptr_t)W & 15);
@@ -374,24 +404,6 @@ static int q_matmul_to(const float *a, const void *W, bool wi8, const float *sca
         Wd = wp;
     }
     const int T = 3;
-    // int8 weights, up to FX_ROWS rows: one full-K launch whose waves split
-    // their k-runs of the f32 rows into int8 terms themselves
-    if (wi8 && m <= FX_ROWS && Wd == W && ((uintptr_t)a & 15) == 0 && k <= (size_t)1 << 30 &&
-        !alias && fx_run_blocks((int)k)) {
-        FxArgs x;
-        x.W = Wsw ? Wsw : Wd;
-        x.swizzled = Wsw != nullptr;
-        x.ldw = (int)k;
-        x.scale = scale;
-        x.X = a;
-        x.ldx = (int)k;
-        x.C = c;
-        x.ldc = (int)n;
-        x.M = (int)m;
-        x.N = (int)n;
-        x.K = (int)k;
-        return launch_fx_gemv(x, st);
-    }
     // int8 weights, a few rows: the wide k-split GEMV splits the f32 rows
     // into terms while staging them, then the slices are reduced in order
     const size_t nch = Kp / 128;
@@ -716,6 +728,8 @@ int vmlm_hip_gemm_nt_int8(const float *a, const int8_t *q, const float *scale, f
     INIT_OR_RETURN();
     VMLM_GUARD(scale != nullptr, "int8 gemm: scale slot must be f32 (null)");
     hipStream_t st = as_stream(stream);
+    int rc;
+    if (q_few_rows(a, q, scale, c, m, n, k, st, nullptr, &rc)) return rc;
     Stage stg(st);
     return q_matmul(a, q, true, scale, c, m, n, k, st, stg);
 }
