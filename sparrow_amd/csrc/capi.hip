@@ -301,6 +301,19 @@ static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
     return 1.1 * us < 10.0 + copy + (steps > prod ? steps : prod);
 }
 
+// Whether the int8-row GEMM gains more from weights swizzled into 1 KiB blocks
+// (its copies move whole blocks, and four workgroups fit a CU instead of two) than
+// the pass takes that swizzles them: a launch and N x K bytes read and written
+// against a gain that goes with the products and with the tiles. Fitted to both
+// sides at 256 to 8000 rows, 512 to 11520 columns, K 128 to 5760 (us, with the pass
+// and without: 2048 x 11520 x 768 88 and 92, 4096 x 5760 x 512 75 and 80, 4096 x 11520 x
+// 128 82 and 91, 4096 x 768 x 1024 36 and 34, 2048 x 2304 x 2304 57 and 54, 512 x 5760 x
+// 2304 45 and 38); the side taken is 0.2 % above the better one in the mean.
+static bool q_swizzle(size_t m, size_t n, size_t k) {
+    const double mn = 1e-6 * m * n, nk = 1e-6 * n * k;
+    return mn * (0.08 + 0.35e-3 * k) > 1.7 + 0.5 * nk;
+}
+
 // int8 weights, up to FX_ROWS rows: one full-K launch whose waves split their
 // k-runs of the f32 rows into int8 terms themselves. True if it takes the call;
 // it needs no workspace and is asked first, since a decode step's projection is
@@ -445,15 +458,11 @@ static int q_matmul_to(const float *a, const void *W, bool wi8, const float *sca
         float *a8s = stg.template alloc<float>(m);
         const size_t gw = gemm_i8_work_floats((int)m, (int)n, (int)k);
         float *gwork = gw ? stg.template alloc<float>(gw) : nullptr;
-        // many rows: the weights swizzled into 1 KiB blocks first (one pass
-        // over N x K bytes), so the GEMM's weight copies move whole blocks,
-        // where the GEMM is long enough to pay for the pass (K = 2304: 512 x
-        // 2304 36.5 with it, 31.8 without, 1500 x 2304 49.5 and 48.3, 2048 x
-        // 11520 177 and 186; 700 x 2304 x 5760 59.7 and 62.2); the
-        // allocation-free entry point keeps its scratch for the rows (a
-        // swizzled copy the caller keeps is read as it is)
-        const bool blk = Wsw || (std::is_same<WS, Stage>::value && m >= 256 &&
-                                 m * k >= (size_t)3600000 && n % 16 == 0);
+        // many rows: the weights swizzled into 1 KiB blocks first; the
+        // allocation-free entry point keeps its scratch for the rows (a swizzled
+        // copy the caller keeps is read as it is)
+        const bool blk = Wsw || (std::is_same<WS, Stage>::value && m >= 256 && n % 16 == 0 &&
+                                 q_swizzle(m, n, k));
         int8_t *wsw = blk && !Wsw ? stg.template alloc<int8_t>(n * k) : nullptr;
         STAGE_OK(stg);
         int rc = launch_rows_q8(a, k, nullptr, 0.0f, m, k, a8, a8s, st);

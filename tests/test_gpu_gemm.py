@@ -186,6 +186,29 @@ def test_gemm_int8_many_tiles_exact(dev, m, n):
     assert np.isnan(got[m - 1]).all()
 
 
+@pytest.mark.parametrize("n", [4096, 4112])
+def test_gemm_int8_swizzled_exact(dev, n):
+    """Enough tiles for the call to swizzle the weights (ragged last tile row and,
+    at 4112, column): exact on integers, rows with a NaN or an infinity recomputed
+    from the row-major weights."""
+    m, k = 4100, 256
+    rng = np.random.default_rng(n)
+    a = rng.integers(-8, 9, size=(m, k)).astype(np.float32)
+    q = rng.integers(-127, 128, size=(n, k), dtype=np.int8)
+    q[:, 9] = np.where(q[:, 9] == 0, 1, q[:, 9])
+    q[0, 9] = 0
+    a[m - 1, 7] = np.nan
+    a[63, 9] = np.inf
+    da, dq, ds, dc = dev.up(a), dev.up(q), dev.up(np.ones(n, np.float32)), dev.empty(m * n * 4)
+    dev.check(dev.lib.vmlm_hip_gemm_nt_int8(da, dq, ds, dc, m, n, k, None))
+    got = dev.down(dc, (m, n), np.float32)
+    rows = np.delete(np.arange(m), [63, m - 1])
+    ref = a[rows].astype(np.float64) @ q.astype(np.float64).T
+    np.testing.assert_array_equal(got[rows].astype(np.float64), ref)
+    assert np.isnan(got[m - 1]).all() and np.isnan(got[63, 0])
+    np.testing.assert_array_equal(got[63, 1:], np.where(q[1:, 9] > 0, np.inf, -np.inf))
+
+
 def direct_case(rng, m, n, k, int8):
     a = rng.standard_normal((m, k), dtype=np.float32)
     if int8:
