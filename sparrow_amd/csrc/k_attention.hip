@@ -1205,7 +1205,9 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(DecodeArgs a, floa
     // Two sub-chunks, the next one's rows requested before each; false: done.
     // A loop's header waits for every load in flight, so the next rows would be
     // requested only when the current ones have arrived: the first four of a
-    // wave are straight code.
+    // wave are straight code. 36 heads, 1024 positions over new caches 10.14 ->
+    // 9.97 us, over the same caches again 7.90 and 8.02; 128 positions 4.00 -> 3.92; a
+    // step at batch 16 equal.
     auto two = [&]() -> bool {
         load(kb, vb, live(s + NW));
         consume(ka, va, s);

@@ -166,8 +166,8 @@ def test_gemm_int8_row_split_wave_path_agrees(dev):
 @pytest.mark.parametrize("m,n", [(2048, 4096),    # 32 x 32 tiles of 64 x 128
                                  (2100, 4112)])   # ragged last tile row and column
 def test_gemm_int8_many_tiles_exact(dev, m, n):
-    """A large grid over blocked weights (M >= 256 swizzles the caller's
-    weights; two LDS stages, four workgroups per CU). Integer activations
+    """A large grid (two LDS stages; the weights as they are, where the pass that
+    swizzles them does not pay). Integer activations
     give exact int8 terms and exact f32 sums, so the result is the float64
     product bit for bit; the ragged case clamps the copies of column tiles
     past the weights and stores only rows < M and columns < N. A NaN row goes
@@ -229,7 +229,9 @@ def test_gemm_direct_edges(dev, m, n, k, int8):
     """Against float64. A result is at most ceil(K / 64 / 4) blocks of two
     MFMAs and three terms in one chain, each MFMA adding 32 products in f32,
     then at most eight waves: the error is within (32 * 6 * ceil(K / 256) + 10)
-    roundings of 2^-24 of sum |a w|."""
+    roundings of 2^-24 of sum |a w|. Roundings of both signs leave far less, 2.5e-7
+    of the result's norm at most; two of the three terms would leave 2.2e-6 or
+    more at each of these sizes (2^-18 of an element), so 5e-7 tells them apart."""
     rng = np.random.default_rng(m + n + k)
     a, w, w64, s = direct_case(rng, m, n, k, int8)
     ref = a.astype(np.float64) @ w64.T
@@ -248,6 +250,29 @@ def test_gemm_direct_edges(dev, m, n, k, int8):
             dev.check(dev.lib.vmlm_hip_gemm_nt_bf16(pa, pw, c, m, n, k, None))
         got = dev.down(c, (m, n), np.float32).astype(np.float64)
         assert (np.abs(got - ref) <= bound).all()
+        assert np.linalg.norm(got - ref) <= 5e-7 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("int8", [True, False])
+@pytest.mark.parametrize("m,n,k", [(2, 17, 63), (17, 40, 577), (33, 2050, 513), (77, 1537, 1001),
+                                   (100, 2304, 5760), (300, 1000, 1000), (12, 9000, 1537)])
+def test_gemm_direct_all_24_bits(dev, m, n, k, int8):
+    """One power of two in each weight row: the product is one row element times
+    it, so all 24 bits of the element come back, each from its term."""
+    rng = np.random.default_rng(m * n + k)
+    a = rng.integers(2 ** 23, 2 ** 24, (m, k)).astype(np.float32) * rng.choice([-1, 1], (m, k))
+    a = (a * 2.0 ** rng.integers(-30, -20, (m, k))).astype(np.float32)
+    at, v = rng.integers(0, k, n), rng.choice([-64, -1, 1, 2, 32], n)
+    w = np.zeros((n, k), np.float32)
+    w[np.arange(n), at] = v
+    c = dev.empty(m * n * 4)
+    if int8:
+        ds = dev.up(np.ones(n, np.float32))
+        dev.check(dev.lib.vmlm_hip_gemm_nt_int8(dev.up(a), dev.up(w.astype(np.int8)), ds, c, m, n,
+                                                k, None))
+    else:
+        dev.check(dev.lib.vmlm_hip_gemm_nt_bf16(dev.up(a), dev.up(bf16_bits(w)), c, m, n, k, None))
+    np.testing.assert_array_equal(dev.down(c, (m, n), np.float32), a[:, at] * v.astype(np.float32))
 
 
 def test_gemm_direct_infinite_and_nan_rows(dev):
@@ -271,8 +296,8 @@ def test_gemm_direct_infinite_and_nan_rows(dev):
 
 
 # int8 rows: rows with a NaN or an infinity written by the GEMM's epilogue (odd N;
-# 96 columns a tile; the swizzled copy) and by the slice reduction; the rows' split
-# in one launch and in two (rows x K past 3.6e6), fewer and more k-slices.
+# 96 columns a tile) and by the slice reduction; the rows' split in one launch and
+# in two (rows x K past 3.6e6), fewer and more k-slices.
 @pytest.mark.parametrize("m,n,k", [(129, 131, 256), (300, 2304, 128), (630, 64, 5760),
                                    (150, 256, 2304), (200, 2048, 4096)])
 def test_gemm_int8_rows_infinite_and_nan_rows(dev, m, n, k):
@@ -295,7 +320,7 @@ def test_gemm_int8_rows_infinite_and_nan_rows(dev, m, n, k):
     # three int8 terms leave at most 2^-21 of the row's maximum per element
     bound = (np.abs(np.where(np.isfinite(a), a, 0)).max(1)[:, None] * 2.0 ** -21 *
              np.abs(w64).sum(1) * s + 1e-5 * np.sqrt(np.mean(ref[ok] ** 2)))
-    assert (np.abs(got.astype(np.float64) - ref)[ok] <= bound[ok]).all()
+    assert (np.abs(got[ok].astype(np.float64) - ref[ok]) <= bound[ok]).all()
 
 
 # f32 GEMM: each tile (32 x 32, 32 x 64, 64 x 64, 128 x 128), rows and columns at
@@ -304,9 +329,8 @@ def test_gemm_int8_rows_infinite_and_nan_rows(dev, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (31, 33, 31), (33, 2305, 96), (40, 100, 1030),
                                    (513, 1028, 64), (1030, 1020, 36), (2049, 2052, 33)])
 def test_gemm_f32_edges(dev, m, n, k):
-    """Against float64: at most ceil(k / 16) chains of four products in one
-    accumulator, then up to 16 slices: (k + 20) roundings of 2^-24 of
-    sum |a b|."""
+    """Against float64: at most k products in one accumulator, then eight of them
+    and up to 16 slices: (k + 20) roundings of 2^-24 of sum |a b|."""
     rng = np.random.default_rng(m + n + k)
     a = rng.standard_normal((m, k), dtype=np.float32)
     b = rng.standard_normal((n, k), dtype=np.float32)
@@ -329,8 +353,7 @@ def test_gemm_f32_edges(dev, m, n, k):
 
 @pytest.mark.parametrize("m,k,int8", [(77, 1001, True), (17, 256, True), (9, 384, False)])
 def test_gemm_over_its_own_rows(dev, m, k, int8):
-    """The result written over the activation rows (n = k): every row is read
-    before the first store, so it is the result in a buffer of its own."""
+    """The result written over the activation rows (n = k), against float64."""
     rng = np.random.default_rng(m * 3 + k)
     a = rng.standard_normal((m, k), dtype=np.float32)
     s = np.full(k, 0.01, np.float32)

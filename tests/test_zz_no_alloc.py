@@ -1,8 +1,8 @@
 """The allocation-free int8 GEMM (vmlm_hip_gemm_nt_int8_noalloc), through the
 C ABI, against the entry point it mirrors (vmlm_hip_gemm_nt_int8). Up to
 M = 255 both run the same kernels. From M = 256 (N a multiple of 16) the
-allocating call first swizzles the weights into 1 KiB blocks in its
-workspace and runs the blocked int8-row GEMM, while the allocation-free call
+allocating call swizzles the weights into 1 KiB blocks in its workspace where that
+pays and runs the blocked int8-row GEMM, while the allocation-free call
 keeps its scratch for the rows and runs the row-major form of the same GEMM
 (its own tile shapes); both sum each term's int8 products exactly in int32
 over the whole K (one k-slice at these grids) and combine them with the same
@@ -82,8 +82,9 @@ def test_noalloc_matches_gemm_nt_int8(dev, oracle):
     run_both(dev, oracle, 3, 1000, 1024, 2)    # smaller, right after
     run_both(dev, oracle, 40, 512, 2304, 3)    # int8 rows + ordered k-slices
     run_both(dev, oracle, 2, 70, 100, 4)       # K % 128 != 0: padded copy in scratch
-    run_both(dev, oracle, 256, 512, 2304, 6)   # M >= 256: blocked (allocating) vs row-major
+    run_both(dev, oracle, 256, 512, 2304, 6)   # M >= 256: row-major in both
     run_both(dev, oracle, 300, 2304, 2304, 7)  # the same with ragged M
+    run_both(dev, oracle, 4100, 4112, 256, 8)  # blocked (allocating) vs row-major
 
 
 def test_noalloc_rejects_oversized(dev):
