@@ -277,18 +277,21 @@ static inline bool overlap(const void *p, size_t np, const void *q, size_t nq) {
 //    equal near 20 us); with more rows it reads the activation again for every
 //    16 columns (16 x 122753 x 2304: 294 -> 108, 16 x 2304 x 2304: 14.3 -> 6.9);
 //  * unpadded int8 at m > 16: int8 rows, the GEMM and the slice reduction are
-//    three launches, 7 + 0.2 per k-step and the products at 500 TFLOP/s (17 x 2304 x 2304: 17.0 -> 7.2; 64 x 5760 x 2304: 21.1 ->
-//    15.8; 100 x 2304 x 5760: 27.6 -> 20.5); up to 128 rows, above which the
-//    row blocks of the int8 GEMM are full (300 x 5760 x 2304: 39 against 44);
+//    three launches, 7 + 0.2 per k-step and the products at 500 TFLOP/s (17 x
+//    2304 x 2304: 16.0 -> 7.7; 64 x 5760 x 2304: 20.5 -> 18; 100 x 2304 x 5760:
+//    26.9 -> 22); up to 128 rows, above which the row blocks of the int8 GEMM are
+//    full (300 x 5760 x 2304: 33 against 49; narrow results stay too: 455 x 236 x
+//    1536 takes 25 so, 7 in one launch);
 //  * else the term planes and the bf16 GEMM: 10, and 0.7 per k-step of one tile
 //    or the products at 230 TFLOP/s; with the padded weight copy the copy at 4
 //    TB/s and, from K = 512, 8 more for its launches (below, the store of C is
 //    much of the direct kernel's time and its estimate too low: 768 x 11520 x 369
-//    int8 stays, 55 to 62) (77 x 1537 x 1001 int8: 30.1 -> 6.6; 1000 x
-//    1500 x 1100: 33.5 -> 22.9; 333 x 1537 x 1536 bf16: 27.5 -> 15.3; 44 x 23698 x
-//    2304 bf16 stays, 34 to 50, and 60 x 40509 x 2304, 66 to 78). The estimate of
-//    the direct kernel is low by a tenth at most sizes near the line (1181 x 1536
-//    x 2328 int8 stays: 56 to 60).
+//    int8 stays, 56 to 64) (77 x 1537 x 1001 int8: 29.4 -> 7.1; 1000 x
+//    1500 x 1100: 35 -> 24; 333 x 1537 x 1536 bf16: 28 -> 18; 44 x 23698 x
+//    2304 bf16 stays, 35 to 50, and 60 x 40509 x 2304, 51 to 66). The estimate of
+//    the direct kernel is low (TILES in k_direct.hip), by a quarter in the middle,
+//    and these lines are drawn where the measured times cross: over 273 sizes drawn
+//    the way taken is 4 % slower than the other at the worst (419 x 5760 x 512 bf16).
 static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
     if (k == 0 || m > 4096 || n > (size_t)1 << 24 || k > (size_t)1 << 24) return false;
     const double us = gemm_direct_us((int)m, (int)n, (int)k, wi8);
@@ -308,7 +311,8 @@ static bool q_direct(bool wi8, bool padded, size_t m, size_t n, size_t k) {
 // sides at 256 to 8000 rows, 512 to 11520 columns, K 128 to 5760 (us, with the pass
 // and without: 2048 x 11520 x 768 88 and 92, 4096 x 5760 x 512 75 and 80, 4096 x 11520 x
 // 128 82 and 91, 4096 x 768 x 1024 36 and 34, 2048 x 2304 x 2304 57 and 54, 512 x 5760 x
-// 2304 45 and 38); the side taken is 0.2 % above the better one in the mean.
+// 2304 45 and 38); the side taken is 0.2 % above the better one in the mean, 9 % at
+// the worst (2048 x 768 x 5760, 71 against 66).
 static bool q_swizzle(size_t m, size_t n, size_t k) {
     const double mn = 1e-6 * m * n, nk = 1e-6 * n * k;
     return mn * (0.08 + 0.35e-3 * k) > 1.7 + 0.5 * nk;

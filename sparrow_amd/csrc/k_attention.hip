@@ -4,7 +4,7 @@
 // -> GEMM NT q.k -> SCALE -> SOFTMAX(causal) -> GEMM NN p.v -> WRITECOL.
 // Here: RoPE is applied once to Q and K (bit-exact port), then one kernel
 // per (head, 64-query block) streams 64-key tiles through LDS with an
-// online softmax (exp_f of the reference, scores scaled exactly as OP_SCALE
+// online softmax (v_exp_f32; scores scaled exactly as OP_SCALE
 // does) -- the [S,S] score matrix never reaches HBM.
 //
 // Decode (tools/p12_build_minicpm.py:941-967): per (sequence, head) one
@@ -16,7 +16,8 @@
 // split over several workgroups, by a second kernel (flash-decoding).
 //
 // Both change the order of the reference's sums (E contract: 1e-4 of the
-// output RMS); RoPE, the scale multiply and every exp_f are bitwise.
+// output RMS); RoPE, the scale multiply and the decode's exp_f are
+// bitwise.
 #include "internal.hpp"
 
 namespace vmlm {
@@ -439,7 +440,7 @@ __device__ __forceinline__ bool prefill_unit(int nqb, int H, int nseq, int causa
 // with the first group (the one-launch kernel's sum, the same bits). Each group
 // copies its tiles straight into its two LDS stages, the next one while the
 // current one is consumed. 36 heads, 1000 causal rows, with the
-// prep launch: 83.6 -> 47 us (2048 rows 244 -> 127).
+// prep launch: 83.6 -> 47 us (2048 rows 244 -> 125).
 constexpr int AT_SPLIT = 4;
 template <int NQ, int NG>
 __global__ __launch_bounds__(256 * NG, 2) void attn_prefill_kernel(PrefillParams P) {

@@ -307,10 +307,14 @@ int launch_tile(const DirectParams &p, hipStream_t st) {
 // on its CU; one block, four waves and half the registers where several
 // workgroups of a large grid hide each other's loads. `lat`, `thr`: us per block
 // of a run with one workgroup on a CU, and per workgroup with its share of the
-// CU full; `res`: workgroups a CU holds (measured at 17 to 1000 rows, 1500 to
-// 11520 columns, K 768 to 5760; the sum below is within 15 % of most of them:
-// 77 x 1537 x 1001 6.6, 64 x 5760 x 2304 15.8, 300 x 5760 x 2304 43.9, 1000 x
-// 1500 x 1100 22.9 us).
+// CU full; `res`: workgroups that share a CU in the fit (at 17 to 1000 rows, 1500
+// to 11520 columns, K 768 to 5760, int8; with bf16 weights LDS holds 1, 3 and 2 of
+// the last three, which would change the choice at 3 of 151 bf16 sizes drawn,
+// slower at two). Over 273 sizes drawn the estimate is 0.55 to
+// 1.05 of the time of a call among others, 0.75 at the median: it lacks the store
+// of C and the rows that every column of tiles reads again (1456 x 2764 x 75 14.4
+// against 21.5 us, 768 x 11520 x 369 41.5 against 64, 100 x 2304 x 5760 20.6 against
+// 21.7). The tile it chooses is 5 % from the best of the seven in the mean.
 struct Tile {
     int tm, tn, nw, res;
     double lat, thr;

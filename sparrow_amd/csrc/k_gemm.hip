@@ -25,8 +25,7 @@ struct GemmParams {
     int group;          // tile order: 0 as dispatched, g > 0 XCD-grouped (gemm_tile)
     int silu;           // int8 rows: C = SiLU(gate) * up of interleaved pairs (GemmArgs)
 };
-// (the other kernel without it: 40 more argument bytes, 6.70 -> 6.79 us at 1024 x
-// 2048 x 512)
+// (the bf16 kernel, whose rows hold whatever they hold, has no use for it)
 struct GemmI8Params : GemmParams {
     NonfiniteRows nf;  // rows with a NaN factor (GemmArgs)
 };

@@ -229,7 +229,7 @@ def test_gemm_direct_edges(dev, m, n, k, int8):
     """Against float64. A result is at most ceil(K / 64 / 4) blocks of two
     MFMAs and three terms in one chain, each MFMA adding 32 products in f32,
     then at most eight waves: the error is within (32 * 6 * ceil(K / 256) + 10)
-    roundings of 2^-24 of sum |a w|. Roundings of both signs leave far less, 2.5e-7
+    roundings of 2^-24 of sum |a w|. Roundings of both signs leave far less, 1.8e-7
     of the result's norm at most; two of the three terms would leave 2.2e-6 or
     more at each of these sizes (2^-18 of an element), so 5e-7 tells them apart."""
     rng = np.random.default_rng(m + n + k)
