@@ -61,12 +61,12 @@ const char *vmlm_hip_version(void);
 int vmlm_hip_sync(void);               /* wait for the library stream */
 int vmlm_hip_malloc(void **dptr, size_t bytes);
 int vmlm_hip_free(void *dptr);
+/* the copies and memset are synchronous, after the library stream's earlier work */
 int vmlm_hip_memcpy_h2d(void *dst, const void *src, size_t bytes);
 int vmlm_hip_memcpy_d2h(void *dst, const void *src, size_t bytes);
-/* device -> device on the library stream (synchronous); also the plain copy
- * of known size that calibrates the HBM traffic counters */
+/* device -> device on the library stream; also the plain copy of known size
+ * that calibrates the HBM traffic counters */
 int vmlm_hip_memcpy_d2d(void *dst, const void *src, size_t bytes);
-/* synchronous, after the library stream's earlier work */
 int vmlm_hip_memset(void *dptr, int value, size_t bytes);
 /* Event timing on a stream (NULL = library stream): returns an opaque id. */
 int vmlm_hip_event_record(void *stream, int *event_id);

@@ -591,6 +591,15 @@ using namespace vmlm;
         return vmlm_hip_check_guards();                   \
     } while (0)
 
+// Waits for what the library stream was given, as a synchronous call on the legacy
+// stream does not; a stream under capture is given nothing.
+static int wait_lib_stream() {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    VMLM_HIP_CHECK(hipStreamIsCapturing(lib_stream(), &cs));
+    if (cs == hipStreamCaptureStatusNone) VMLM_HIP_CHECK(hipStreamSynchronize(lib_stream()));
+    return VMLM_OK;
+}
+
 extern "C" {
 
 // ================================================================ library
@@ -621,6 +630,8 @@ int vmlm_hip_free(void *dptr) {
 }
 int vmlm_hip_memcpy_h2d(void *dst, const void *src, size_t bytes) {
     INIT_OR_RETURN();
+    const int rc = wait_lib_stream();  // its queued calls may still read dst
+    if (rc) return rc;
     VMLM_HIP_CHECK(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
     return VMLM_OK;
 }
@@ -640,11 +651,10 @@ int vmlm_hip_memset(void *dptr, int value, size_t bytes) {
     INIT_OR_RETURN();
     // hipMemset runs on the legacy stream, which neither waits for the
     // library's non-blocking stream nor is waited for by it, and may return
-    // before the memory is set: after what the library stream was given (a
-    // stream under capture is given nothing), and before what it is given next
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    VMLM_HIP_CHECK(hipStreamIsCapturing(lib_stream(), &cs));
-    if (cs == hipStreamCaptureStatusNone) VMLM_HIP_CHECK(hipStreamSynchronize(lib_stream()));
+    // before the memory is set: after what the library stream was given, and
+    // before what it is given next
+    const int rc = wait_lib_stream();
+    if (rc) return rc;
     VMLM_HIP_CHECK(hipMemset(dptr, value, bytes));
     VMLM_HIP_CHECK(hipStreamSynchronize(nullptr));
     return VMLM_OK;

@@ -487,3 +487,18 @@ def test_gemm_f32_sums_in_short_runs(dev, m, n, k):
         dev.check(f(da, db, c, m, n, k, False, None))
         got = dev.down(c, (m, n), np.float32).astype(np.float64)
         assert np.abs(got - (1 + (k - 1) * 2.0 ** -25)).max() <= (run + 2 * (3 + slices)) * 2.0 ** -25
+
+
+def test_upload_after_queued_work(dev):
+    """memcpy_h2d comes after the calls that still read what it writes over."""
+    n = 2048
+    rng = np.random.default_rng(5)
+    a, b = (rng.standard_normal((n, n), dtype=np.float32) for _ in range(2))
+    da, one = dev.up(a), dev.up(np.eye(n, dtype=np.float32))
+    cs = [dev.empty(n * n * 4) for _ in range(8)]
+    for c in cs:
+        dev.check(dev.lib.vmlm_hip_gemm_nt(da, one, c, n, n, n, False, None))
+    dev.check(dev.lib.vmlm_hip_memcpy_h2d(da, b.ctypes.data, b.nbytes))
+    for c in cs:
+        assert np.array_equal(dev.down(c, (n, n), np.float32), a)
+    assert np.array_equal(dev.down(da, (n, n), np.float32), b)
