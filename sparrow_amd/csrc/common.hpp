@@ -391,7 +391,8 @@ constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (0x7 << 
 // waits and publish them with barriers. m0 is not used by anything else in
 // the kernels that use these. A write of m0 needs one wait state before a load
 // into LDS reads it; the compiler fills none inside an assembly string, so the
-// s_nop is part of it.
+// s_nop is part of it (under 1 % of the kernels' time: 1000 x 2304 x 2304 f32 112.9 us
+// without it, 113.7 with it; 1024 x 2048 x 512 bf16 6.7 and 6.7).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved; nothing else here uses it
 __device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_base) {
